@@ -1,0 +1,67 @@
+"""Which block runs which tile of a grouped GEMM: row counts at the edges of the tile classes (32 | 33, 128 | 129,
+383 | 384 rows), with and without heavy experts, more and fewer tiles than blocks.  A schedule that drops, repeats or
+misplaces a tile leaves wrong rows: the chained launch is compared bit for bit with the two calls (themselves compared
+with the oracle in test_gpu_gmm.py), the int8 GEMM with its exact integer sums."""
+import pytest
+import torch
+
+from test_gpu_chain import DT_BF16, DT_FP8, Case, lib  # noqa: F401 (lib is a fixture)
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [32, 33, 128, 129, 383, 1, 0, 64]
+PREFILL = [
+    (EDGES, 2048, 2048),                                # no heavy expert
+    (EDGES + [384], 2048, 2048),                        # heavy tiles on some blocks, the others free at once
+    ([384, 700] * 9 + EDGES, 2048, 2048),               # more heavy tiles than blocks
+    ([40, 20, 130] * 12, 2048, 2048),                   # several rounds of light tiles through the queue
+    (EDGES, 256, 384),                                  # reductions of 2 and 3 k-steps: no tile primes the next
+]
+
+
+@pytest.mark.parametrize("dt", [DT_FP8, DT_BF16])
+@pytest.mark.parametrize("case", range(len(PREFILL)))
+def test_chained_prefill_tiles_at_class_edges(lib, dt, case):  # noqa: F811
+    counts, H, I = PREFILL[case]
+    print(f"chained schedule counts={counts} dt={dt}", flush=True)
+    c = Case(counts, H, I, dt, 50 + case)
+    assert c.cap > 48 * c.L or case == 3  # the 8-wave kernel (and once the 4-wave one with two tiles per expert)
+    for _ in range(2):
+        c.new_outputs()
+        c.run_pair(lib)
+        c.run_chain(lib)
+        c.assert_same()
+    assert lib.sync_status() == 0
+
+
+@pytest.mark.parametrize("counts", [[1, 0, 1, 0, 0, 0, 0, 0], [0, 3], [33, 1, 32, 40], [1] * 40])
+@pytest.mark.parametrize("dt", [DT_FP8, DT_BF16])
+def test_chained_decode_few_tiles(lib, dt, counts):  # noqa: F811
+    # fewer GMM2 tiles than blocks without GMM1 work: they spread over the free blocks
+    print(f"chained decode counts={counts} dt={dt}", flush=True)
+    c = Case(counts, 1024, 512, dt, 70)
+    c.run_pair(lib)
+    c.run_chain(lib)
+    c.assert_same()
+    assert lib.sync_status() == 0
+
+
+@pytest.mark.parametrize("counts", [EDGES, EDGES + [384, 900], [2100, 40, 2100, 150, 3, 129, 128]])
+def test_int8_tiles_at_class_edges(counts):
+    # int8 x int8 sums in fp64 are exact (|sum| < 2^53), then the kernel's own fp32 sequence and bf16 rounding
+    import umdk_amd  # noqa: F401
+    print(f"int8 schedule counts={counts}", flush=True)
+    L, M, H, I = len(counts), sum(counts), 4096, 2048
+    g = torch.Generator(device="cuda").manual_seed(len(counts))
+    x = torch.randint(-127, 128, (M, I), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (L, H, I), dtype=torch.int8, device="cuda", generator=g)
+    xs = torch.rand(M, device="cuda", generator=g) * 0.01
+    ws = torch.rand(L, H, device="cuda", generator=g) * 0.01
+    gl = torch.tensor(counts, dtype=torch.int64, device="cuda")
+    y = torch.ops.umdk_cam_op_lib.grouped_matmul(x, xs, gl, w, ws)
+    at = 0
+    for e, n in enumerate(counts):
+        acc = x[at:at + n].double() @ w[e].double().T
+        ref = ((acc.float() * ws[e]) * xs[at:at + n, None]).bfloat16()
+        assert torch.equal(y[at:at + n].view(torch.int16), ref.view(torch.int16)), f"expert {e} of {n} rows"
+        at += n

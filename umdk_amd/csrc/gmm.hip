@@ -65,9 +65,6 @@ typedef __attribute__((ext_vector_type(8))) int i32x8;
 // 1.31 vs 1.27 PFLOPS, config 4's 278-284 vs 286 us; fewer address and scalar instructions per k-step)
 #define CAM_GMM_UNROLL2 1
 #endif
-#ifndef CAM_GMM_NT_MAXBM
-#define CAM_GMM_NT_MAXBM 32  // tile heights up to this stream their weights nontemporally
-#endif
 
 constexpr int GBN = 256, GKB = 128;  // tile W-rows, bytes per row per k-step
 constexpr int GMAX_THREADS = 512;    // block size of the largest tile
@@ -107,14 +104,28 @@ template <int BM_, int BN_ = GBN> struct Tile {
 #endif
 constexpr int small_bn(int bm, int epi) { return bm == 32 && epi == 0 ? CAM_GMM_SMALL_PLAIN_BN : GBN; }
 
-// Expert tables of a launch, built once at kernel start: per tile class (256-, 128- and 32-row tiles) the
-// inclusive prefix of M-tiles per expert, and the inclusive prefix of rows per expert (the exclusive prefix
-// of expert e is entry e-1, or 0 for e = 0; no entry for it keeps the tables within the LDS budget).
-constexpr int G_NCLASS = 3;
-constexpr int tile_class(int bm) { return bm >= 256 ? 0 : bm >= 128 ? 1 : 2; }
+// Tile classes: 256-row tiles, 128-row tiles of experts with several of them, 128-row tiles of experts with one,
+// 32-row tiles.  The two 128-row classes differ in how they fetch their weights (see W_CACHED and W_STREAM).
+enum TileClass { CLS_256 = 0, CLS_128M = 1, CLS_128S = 2, CLS_32 = 3 };
+constexpr int G_NCLASS = 4;
+constexpr int class_bm(int cls) { return cls == CLS_256 ? 256 : cls == CLS_32 ? 32 : 128; }
+
+// Expert tables of a launch, built once at kernel start: per tile class the inclusive prefix of M-tiles per
+// expert, and the inclusive prefix of rows per expert (the exclusive prefix of expert e is entry e-1, or 0 for
+// e = 0; no entry for it keeps the tables within the LDS budget).  The last two classes share a word: at most one
+// tile per expert in CLS_128S (<= 512), and CLS_32 only ever takes experts of fewer than G_SMALL_ROWS rows or a
+// launch of at most 48 rows per expert (<= 1280 tiles).
 struct GroupTables {
-    int tile_end[G_NCLASS][G_MAX_L];
+    int tile_end[G_NCLASS - 2][G_MAX_L];
+    uint32_t tile_end_s[G_MAX_L];  // CLS_128S << 16 | CLS_32
     int row_end[G_MAX_L];
+    template <int CLS> __device__ __forceinline__ int end(int e) const
+    {
+        if constexpr (CLS < CLS_128S)
+            return tile_end[CLS][e];
+        else
+            return CLS == CLS_128S ? (int)(tile_end_s[e] >> 16) : (int)(tile_end_s[e] & 0xffffu);
+    }
 };
 // the experts each class takes: a row count in [lo, hi) (lo >= hi: the class is not used)
 struct ClassRanges {
@@ -150,10 +161,10 @@ __device__ __forceinline__ const ChainParams *chain_params()
     return (const ChainParams *)(const __attribute__((address_space(4))) ChainParams *)a;
 }
 
-// readiness counters of a chained launch: the M-tiles (at most M/32 + L), then one arrival counter per XCD,
-// then one heavy-tile queue per XCD
-__host__ __device__ constexpr int chain_arrival_index(int M, int L) { return M / 32 + L + 1; }
-__host__ __device__ constexpr int chain_queue_index(int M, int L) { return chain_arrival_index(M, L) + 8; }
+// readiness counters of a chained launch: the M-tiles (at most M/32 + L), then the tile queues of the 8-wave kernel:
+// GMM2's heavy tiles (one queue per XCD), the light tiles of GMM1 and of GMM2
+__host__ __device__ constexpr int chain_queue_index(int M, int L) { return M / 32 + L + 1; }
+__host__ __device__ constexpr int chain_light_index(int M, int L, bool gmm2) { return chain_queue_index(M, L) + 8 + gmm2; }
 
 // h stores of a producing GMM1 tile: agent-coherent (sc1, written through to memory), so that a GMM2 tile on
 // another XCD, whose L2 has never held these lines during the launch, reads them from memory
@@ -203,27 +214,44 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // dispatch order).
 template <int GTHREADS>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
-                                   const ClassRanges &cr)
+                                   ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{})
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
-    constexpr int BMS[G_NCLASS] = {256, 128, 32};
+    constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(1), class_bm(2), class_bm(3)};
     const int tid = threadIdx.x;
     const int per = (L + GTHREADS - 1) / GTHREADS;
-    int cnt[4] = {0, 0, 0, 0};
+    constexpr int NWV = GTHREADS / 64;
+    const int lane = tid & 63, wv = tid >> 6;
+    int cnt[NQ] = {};
     auto add = [&](int c, int *v) {
 #pragma unroll
         for (int k = 0; k < G_NCLASS; ++k)
             v[k] += (c >= cr.lo[k] && c < cr.hi[k]) ? (c + BMS[k] - 1) / BMS[k] : 0;
         v[G_NCLASS] += c;
     };
+    if (heavy_rows > 0) {  // cr_heavy where some expert holds that many rows
+        int any = 0;
+        for (int q = 0; q < per; ++q)
+            any |= tid * per + q < L && group_list[tid * per + q] >= heavy_rows;
+        int *flag = scratch + NQ * NWV;
+        if (lane == 0)
+            flag[wv] = 0;
+        if (any)
+            flag[wv] = 1;
+        __syncthreads();
+        any = 0;
+#pragma unroll
+        for (int v = 0; v < NWV; ++v)
+            any |= flag[v];
+        if (any)
+            cr = cr_heavy;
+    }
     for (int q = 0; q < per; ++q) {
         const int e = tid * per + q;
         if (e < L)
             add((int)group_list[e], cnt);
     }
     // exclusive scan: within each wave by lane shuffles, then over the waves' totals
-    constexpr int NWV = GTHREADS / 64;
-    const int lane = tid & 63, wv = tid >> 6;
     int inc[NQ];
 #pragma unroll
     for (int k = 0; k < NQ; ++k)
@@ -256,9 +284,9 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
         const int e = tid * per + q;
         if (e < L) {
             add((int)group_list[e], run);
-#pragma unroll
-            for (int k = 0; k < G_NCLASS; ++k)
-                gt.tile_end[k][e] = run[k];
+            gt.tile_end[CLS_256][e] = run[CLS_256];
+            gt.tile_end[CLS_128M][e] = run[CLS_128M];
+            gt.tile_end_s[e] = (uint32_t)run[CLS_128S] << 16 | (uint32_t)run[CLS_32];
             gt.row_end[e] = run[G_NCLASS];
         }
     }
@@ -272,6 +300,15 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * GKB + ((ch
 
 // the lane's index in its wave, from mbcnt (no work-item id register)
 __device__ __forceinline__ int lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
+// the same, recomputed where it stands: what a tile switch derives from the lane is then not kept in registers through
+// the k-loop (which spills it, each reload waiting for every store of the epilogue before it)
+__device__ __forceinline__ int lane_here()
+{
+    int l = lane_id();
+    asm volatile("" : "+v"(l));
+    return l;
+}
 
 // s_waitcnt with only vmcnt constrained (expcnt and lgkmcnt at their maxima)
 template <int N> __device__ __forceinline__ void wait_vmcnt()
@@ -361,18 +398,33 @@ __device__ __forceinline__ void lds_sync()
 // sy.ready; SYNC_CONSUME tiles start their DMAs only once sy.ready of their M-tile has reached sy.target.  Waves
 // beyond the tile's own (a 32-row class run by an 8-wave block) are spectators: they issue no DMA, MFMA or store
 // and only meet the block's barriers.
-constexpr int G_DYN = -2;  // gmm_body's `first` for a dynamic tile queue (see there)
+// A dynamic tile queue: tickets off, off + 1, ... handed out one at a time by the counter SY().ready[ctr]; ticket t
+// of [base, end) is tile first + t - base of the class at hand.  tk: the block's first ticket, -1 to take one.
+struct TileQueue {
+    int ctr, off, base, end, first, tk;
+};
 
 // EAGER (the 4-wave chained kernel): a producer's primed tile counts its predecessor at k-step edge STAGES-2
-// instead of after its k-loop (a branch inside the k-loop, which the 8-wave kernels cannot afford).  bid: the
-// block's position for balanced placement (a chained consumer passes its arrival order), -1: blockIdx.x.
+// instead of after its k-loop (a branch inside the k-loop, which the 8-wave kernels cannot afford).
 // wv: the wave's index in the block (a scalar the kernel computes once; -1: from threadIdx.x).  The body
 // takes the lane from mbcnt and never reads the work-item id: a register holding it through the whole kernel
 // gets spilled, and each reload before a k-loop makes the loop wait for it at every iteration.
-template <int DT, int EPI, int BM, bool NTW = (BM <= CAM_GMM_NT_MAXBM), int ROLE = SYNC_NONE, bool EAGER = false>
-__device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gtab, int first, int rs = 0, int rn = 0,
-                                         int rstride = 1, int bid = -1, int wv = -1)
+// How a tile fetches its weights: cached, nontemporally, or either by the number of the expert's M-tiles (a k-loop for
+// each: the 8-wave kernels have no registers for that).  An expert that fits one M-tile has its weights read exactly
+// once; the M-tiles of an expert of several, which the tile order runs side by side on one XCD, re-read them from that
+// XCD's L2 (48 experts of 36 to 281 rows, fp8, K = 4096, N = 2816: 173 us cached, 205 us nontemporal).  A stream past
+// the caches pays where it spares the L2 lines that others re-read: the 4-wave decode tiles, and the single M-tiles
+// beside heavy experts (the int8 layer of 22 touched experts, one of 2311 rows: 382 us nontemporal, 405 us cached);
+// without heavy experts cached weights are as fast with many tiles (160 against 158 us for 48 experts of 100 rows) and
+// faster with few (54 against 60 us for one expert of 128 rows, N = 4096, K = 7168).
+enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
+constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? W_STREAM : W_CACHED; }
+
+template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS)>
+__device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gtab, int first, int rs = 0, int rn = 0,
+                                        int rstride = 1, int wv = -1, const TileQueue &tq = TileQueue{})
 {
+    constexpr int BM = class_bm(CLS);
     using TC = Tile<BM, small_bn(BM, EPI)>;
     constexpr int TBN = TC::BN;
     constexpr int NW = TC::NWAVES;
@@ -382,8 +434,8 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     // the epilogue's exchange area (fp8 amax, int8 row maxima) follows this class's ring
     int *scratch = reinterpret_cast<int *>(smem + GSTAGES * STAGE_BYTES);
-    const int *tile_end = gtab->tile_end[tile_class(BM)];
-    auto tile_prefix = [&](int e) { return e > 0 ? tile_end[e - 1] : 0; };
+    auto tile_end = [&](int e) { return gtab->template end<CLS>(e); };
+    auto tile_prefix = [&](int e) { return e > 0 ? tile_end(e - 1) : 0; };
     auto row_off = [&](int e) { return e > 0 ? gtab->row_end[e - 1] : 0; };
 
     const int lane = lane_id();
@@ -396,9 +448,12 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
     // M-tiles of the classes before this one (the readiness counters' index base), read when needed
     auto cls_base = [&]() {
         int b = 0;
-#pragma unroll
-        for (int k = 0; k < tile_class(BM); ++k)
-            b += gtab->tile_end[k][p.L - 1];
+        if constexpr (CLS > CLS_256)
+            b += gtab->template end<CLS_256>(p.L - 1);
+        if constexpr (CLS > CLS_128M)
+            b += gtab->template end<CLS_128M>(p.L - 1);
+        if constexpr (CLS > CLS_128S)
+            b += gtab->template end<CLS_128S>(p.L - 1);
         return __builtin_amdgcn_readfirstlane(b);
     };
     constexpr bool SWIGLU = EPI != EPI_PLAIN;
@@ -417,15 +472,18 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
     // stream is bound by aggregate HBM bandwidth, which that many CUs still saturate, and no CU is left
     // streaming a final partial round alone.  Otherwise the caller's position and the full grid stride.
     int G = gridDim.x, logical = first;
-    // G_DYN (chained consumer, 256-row tiles): tiles rs, rs + 1, ... rs + rn - 1 handed out one at a time by
-    // the queue counter SY().ready[rstride], shared by the blocks of one XCD
-    const bool dyn = CONSUME && BM >= 256 && first == G_DYN;
+    // tiles from the queue tq, in the 8-wave chained kernel: the consumer's heavy tiles (a queue per XCD) and the
+    // light tiles of both GEMMs
+    constexpr bool dyn = CONSUME && BM >= 256;
+    constexpr bool DYNL = ROLE != SYNC_NONE && BM < 256 && !EAGER;
+    int tk = tq.tk;
+    auto ticket_tile = [&](int t) { return t < tq.end ? tq.first + t - tq.base : 0x7fffffff; };
     if (first == -1) {
-        const int b = bid >= 0 ? bid : (int)blockIdx.x;
+        const int b = blockIdx.x;
         const int rounds = max((total + G - 1) / G, 1);
         const int g_eff = min(G, ((total + rounds - 1) / rounds + 7) / 8 * 8);
         if (b >= g_eff)
-            return;
+            return tk;
         G = g_eff;
         logical = (b & 7) * (G >> 3) + (b >> 3);
     }
@@ -434,8 +492,6 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
 
     // DMA slot of this lane inside a 1 KiB band (8 rows x 128 B): row l/8, physical chunk l%8,
     // which holds logical chunk (l%8) ^ ((row >> 1) & 7) -- see swz()
-    const int band_row = lane >> 3;
-    auto chunk_off = [&](int r) { return (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4); };
 
     // ---- one tile's coordinates and the per-lane sources of this wave's DMA bands
     struct Ctx {
@@ -445,19 +501,22 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         uint32_t ga[A_LOADS], gb[B_LOADS], gs[TC::S_DMAS];
         int wsg, wsu;  // fp8: weight-scale row offsets (gate / up n-blocks, or the wave's column block)
         int active;    // some row of this wave lies inside the segment (an int: a bool tail makes struct copies go through scratch)
+        int nt;        // the expert's only M-tile (W_BY_TILE)
     };
     auto setup = [&](int tile, Ctx &c) {
+        const int lane = lane_here(), band_row = lane >> 3;
+        auto chunk_off = [&](int r) { return (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4); };
         int lo = 0, hi = p.L - 1;
         while (lo < hi) {  // last e with tile_prefix[e]*ntn <= tile
             const int mid = (lo + hi + 1) >> 1;
-            if (tile_end[mid - 1] * ntn <= tile)
+            if (tile_end(mid - 1) * ntn <= tile)
                 lo = mid;
             else
                 hi = mid - 1;
         }
         const int e = __builtin_amdgcn_readfirstlane(lo);
         c.e = e;
-        const int mt_e = __builtin_amdgcn_readfirstlane(tile_end[e] - tile_prefix(e));
+        const int mt_e = __builtin_amdgcn_readfirstlane(tile_end(e) - tile_prefix(e));
         const int local = __builtin_amdgcn_readfirstlane(tile - tile_prefix(e) * ntn);
         // within the expert: groups of up to 8 M-tiles, N-tiles in turn, the group's M-tiles
         // fastest -- a run of consecutive tiles (one XCD's share of a round) covers ~8 A row blocks
@@ -473,6 +532,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         // a wave whose rows all lie past the segment skips its MFMAs (it still moves its share of the
         // DMA and meets every barrier): a tile of a short segment costs little more than its weights
         c.active = !spect && c.row0 + wm * WM < c.seg1;
+        c.nt = mt_e == 1;
 
         if (p.Wl) {  // separated weights: one allocation per expert, pointers read by scalar loads (a vector
                      // load here would make the tile switch wait for every DMA in flight)
@@ -518,8 +578,9 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         c.wsu = SWIGLU ? ((half_n + c.n0) / 128) * nk : c.wsg;
     };
     // DMA instruction q (0 <= q < LOADS) of k-step kc of tile c into ring slot `slot`: A bands, then
-    // W bands, then (fp8) the activation scales
-    auto dma_one = [&](const Ctx &c, int kc, int slot, int q) {
+    // W bands (nt: nontemporally), then (fp8) the activation scales
+    auto dma_one = [&](const Ctx &c, int kc, int slot, int q, auto nt) {
+        constexpr bool NTW = decltype(nt)::value;
         if (spect)
             return;
         uint8_t *st = smem + slot * STAGE_BYTES;
@@ -541,9 +602,6 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             dma16(p.A + c.ga[q] + (uint32_t)kc * GKB, st + (q * NW + w) * 1024);
         } else if (q < A_LOADS + B_LOADS) {
             const int i = q - A_LOADS;
-            // decode tiles and the light experts' tiles of a skewed prefill launch (NTW): the weights are a
-            // stream read about once, fetched nontemporally (measured: the config-5 decode step 244 vs
-            // 274 us, config 4's GMM1 216 vs 222 us)
             if constexpr (NTW)
                 dma16_nt(c.wbase + c.gb[i] + (uint32_t)kc * GKB, st + A_BYTES + (i * NW + w) * 1024);
             else
@@ -587,6 +645,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             return;
         }
         const int row0 = c.row0, seg1 = c.seg1, n0 = c.n0;
+        const int lid = lane_here(), l16 = lid & 15, lg = lid >> 4;
         if constexpr (EPI == EPI_PLAIN) {
 #pragma unroll
             for (int i = 0; i < IF; ++i) {
@@ -660,11 +719,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                 }
             } else {
                 // fp8 1x128 requant: the tile's 128 h-columns of a row are one scale block,
-                // split over the column waves; exchange partial amax through LDS.  The lane's row and
-                // column offsets are recomputed here from the lane id (mbcnt): values kept from the kernel's
-                // start are spilled by the k-loop, and each reload would wait on every store issued before it
-                const int lid = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-                const int l16 = lid & 15, lg = lid >> 4;
+                // split over the column waves; exchange partial amax through LDS
                 float *red = reinterpret_cast<float *>(scratch);  // [WAVES_N][GBM]
 #pragma unroll
                 for (int i = 0; i < IF; ++i) {
@@ -723,6 +778,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
     // v = ((float)acc * w_scale[n]) * x_scale[m]  (block_epilogue_per_token_dequant*.h)
     auto dequant_int8 = [&](const Ctx &cur) {
         if constexpr (INT8) {
+            const int lid = lane_here(), l16 = lid & 15, lg = lid >> 4;
             const float *wsr = cur.wsb;
 #pragma unroll
             for (int j = 0; j < JF; ++j) {
@@ -785,12 +841,31 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             }
         }
     };
+    // a queue's next ticket: thread 0 takes it and publishes it to the block through the epilogue's exchange area
+    // (a second barrier when the epilogue that follows writes there)
+    auto take = [&]() -> int {
+        int t = 0;
+        if constexpr (CONSUME || DYNL) {
+            if (first_thread)
+                t = tq.off + __hip_atomic_fetch_add(gptr(SY().ready + tq.ctr), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        return t;
+    };
+    auto publish = [&](int t) -> int {
+        if (first_thread)
+            scratch[0] = t;
+        lds_sync();
+        t = __builtin_amdgcn_readfirstlane(scratch[0]);
+        if constexpr (EPI != EPI_PLAIN)
+            lds_sync();
+        return t;
+    };
     // the M-tile counter of a tile index (the expert search of setup, nothing else)
     auto mti_of = [&](int tile) {
         int lo = 0, hi = p.L - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
-            if (tile_end[mid - 1] * ntn <= tile)
+            if (tile_end(mid - 1) * ntn <= tile)
                 lo = mid;
             else
                 hi = mid - 1;
@@ -798,7 +873,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         const int e = __builtin_amdgcn_readfirstlane(lo);
         const int local = tile - tile_prefix(e) * ntn;
         constexpr int GM = 8;
-        const int mt_e = tile_end[e] - tile_prefix(e);
+        const int mt_e = tile_end(e) - tile_prefix(e);
         const int grp = local / (GM * ntn), rem = local % (GM * ntn);
         const int gm = min(GM, mt_e - grp * GM);
         return __builtin_amdgcn_readfirstlane(cls_base() + tile_prefix(e) + grp * GM + rem % gm);
@@ -823,35 +898,19 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         auto prime = [&](const Ctx &c) {
 #pragma unroll
             for (int q = A_LOADS; q < A_LOADS + B_LOADS; ++q)
-                dma_one(c, 0, 0, q);
+                dma_one(c, 0, 0, q, std::false_type{});
 #pragma unroll
             for (int q = 0; q < LOADS; ++q)
                 if (q < A_LOADS || q >= A_LOADS + B_LOADS)
-                    dma_one(c, 0, 0, q);
+                    dma_one(c, 0, 0, q, std::false_type{});
 #pragma unroll
             for (int q = A_LOADS; q < A_LOADS + B_LOADS; ++q)
-                dma_one(c, min(1, nk - 1), 1, q);
-        };
-        // dynamic queue: thread 0 takes the next index and publishes the tile through the (plain-epilogue,
-        // so unused) exchange area; past the queue's end, `total`
-        int *qslot = reinterpret_cast<int *>(scratch) + 128;
-        auto take = [&]() {
-            if constexpr (CONSUME) {
-                return __hip_atomic_fetch_add(gptr(SY().ready + rstride), 1, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-            }
-            return 0;
-        };
-        auto publish = [&](int k) {
-            if (first_thread)
-                *qslot = k < rn ? rs + k : total;
-            lds_sync();
-            return __builtin_amdgcn_readfirstlane(*qslot);
+                dma_one(c, min(1, nk - 1), 1, q, std::false_type{});
         };
         int kt = 0, tile;
         if (dyn) {
-            const int k = first_thread ? take() : 0;
-            tile = publish(k);
+            tk = publish(take());
+            tile = min(ticket_tile(tk), total);
         } else {
             tile = seq(0);
         }
@@ -964,13 +1023,13 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                             if (n < HALF) {
 #pragma unroll
                                 for (int u = n * AS / HALF; u < (n + 1) * AS / HALF; ++u)
-                                    dma_one(c, kn, 1 - SL, u < A_LOADS ? u : u + B_LOADS);
+                                    dma_one(c, kn, 1 - SL, u < A_LOADS ? u : u + B_LOADS, std::false_type{});
                             }
                             if (n == HALF) {
                                 bar();
 #pragma unroll
                                 for (int q = A_LOADS; q < A_LOADS + B_LOADS; ++q)
-                                    dma_one(c, min(ks + 2, nk - 1), SL, q);
+                                    dma_one(c, min(ks + 2, nk - 1), SL, q, std::false_type{});
                             }
                             if constexpr (FP8) {
                                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
@@ -1012,9 +1071,10 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             if (dyn) {
                 // the queue's answer arrives while the ring drains; then the next tile's counter, answered
                 // during the epilogue
-                const int k = first_thread ? take() : 0;
+                const int t = take();
                 wait_vmcnt<0>();
-                ntile = publish(k);
+                tk = publish(t);
+                ntile = min(ticket_tile(tk), total);
                 if (ntile < total && !gave_up)
                     next_ready = poll(mti_of(ntile));
             } else {
@@ -1051,7 +1111,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             bar();
             signal();
         }
-        return;
+        return tk;
     } else {
         // ---- 128/32-row tiles: software-pipelined k-loop over a ring of STAGES slots, continued
         // across the block's tiles.  Ring slots are indexed by the block's running k-step count kb+ks,
@@ -1060,10 +1120,19 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         // with its operands already in flight.  With fewer k-steps than stages, or no next tile, the
         // past-the-end DMAs reload the tile's last k-step (the DMA count per k-step, and so every
         // vmcnt wait, stays uniform) and the ring is drained before the next tile.
-        int kt = 0;
-        int tile = seq(0);
+        int kt = 0, tile;
+        if constexpr (DYNL) {
+            // Light tiles of the 8-wave chained kernel: taken from the queue only when the block is free, so that
+            // no block ends a GEMM more than one light tile after the others.  The next tile's DMAs start between
+            // this one's drained ring and its epilogue.
+            if (tk < 0)
+                tk = publish(take());
+            tile = ticket_tile(tk);
+        } else {
+            tile = seq(0);
+        }
         if (tile >= total)
-            return;
+            return tk;
         Ctx cur, nxt;
         setup(tile, cur);
         CAM_TL_DECL
@@ -1071,27 +1140,16 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
         bool primed = false;  // the current tile's first STAGES k-steps were issued by the previous tile
         int cur_ready = 0;    // consumer: the current tile's counter as polled before the previous tile's epilogue
         const bool can_chain = nk >= GSTAGES && (!(CONSUME && EAGER) || nk >= 2 * GSTAGES - 2);
-        // A consumer chains into its next tile only when that tile's rows are ready.  Nothing of this runs
-        // inside the k-loop (a branch there makes the compiler duplicate the loop): wave 0 copies the counter
-        // of the tile after next into an LDS slot by DMA at each tile's start, and every wave reads the next
-        // tile's slot after the tile's first barrier -- the copy was issued a whole tile earlier, and that
-        // tile's k-step waits have covered it.  The block's second tile's counter is copied before its first
-        // tile's DMAs.  Two slots of 64 ints (a DMA writes one per lane) in the exchange area, which the plain
-        // epilogue does not use; tile k's counter goes to slot k & 1.
-        int *rslot = scratch;
-        // EAGER consumer (the 4-wave kernel, which affords a branch in its k-loop): the copy goes out at k-step
-        // edge nk - 2 STAGES + 2 and is read at edge nk - STAGES, just before the first past-the-end DMA, so the
-        // decision uses a counter value from late in the current tile
+        // A consumer of the 4-wave kernel chains into its next tile only when that tile's rows are ready: wave 0
+        // copies the tile's counter into LDS by DMA at k-step edge nk - 2 STAGES + 2 (into the exchange area, which
+        // the plain epilogue does not use), and every wave reads it at edge nk - STAGES, just before the first
+        // past-the-end DMA.  (The 8-wave kernel cannot afford that branch in its k-loop; its light tiles do not
+        // chain.)
         constexpr bool EAGER_C = CONSUME && EAGER;
         const int e_copy = nk - 2 * GSTAGES + 2, e_read = nk - GSTAGES;
-        if constexpr (CONSUME && !EAGER) {
-            const int t1 = seq(1);
-            if (t1 < total && w == 0)
-                dma4_sc1(SY().ready + mti_of(t1), rslot + 64);
-        }
         while (true) {
-            const int ntile = seq(++kt);
-            const bool has_next = ntile < total;
+            int ntile = DYNL ? total : seq(++kt);
+            bool has_next = ntile < total;
             // (int8 chains too: its dequantisation's vector loads then wait for the next tile's first DMAs,
             // which land meanwhile -- measured 8 us faster on the int8 decode step than draining first)
             int chain = has_next && can_chain;
@@ -1101,33 +1159,45 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                 nxt = cur;
             auto slot = [&](int ks) { return (kb + ks) % GSTAGES; };
             auto stage_ptr = [&](int ks) { return smem + slot(ks) * STAGE_BYTES; };
-            // DMA instruction q of the current tile's k-step ksx (ksx may run past the end)
-            auto dma_ks = [&](int ksx, int q) {
+            // DMA instruction q of the current tile's k-step ksx (ksx may run past the end: the next tile's first
+            // k-steps go out under the current tile's cache policy)
+            auto dma_ks = [&](int ksx, int q, auto nt) {
                 // a uniform branch between two direct calls: selecting the context by reference would
                 // place one of them in scratch memory, and every reload from there waits for the whole
                 // DMA ring (vmcnt(0))
                 if (ksx >= nk && chain)
-                    dma_one(nxt, ksx - nk, slot(ksx), q);
+                    dma_one(nxt, ksx - nk, slot(ksx), q, nt);
                 else
-                    dma_one(cur, min(ksx, nk - 1), slot(ksx), q);
+                    dma_one(cur, min(ksx, nk - 1), slot(ksx), q, nt);
             };
             // the DMAs that follow MFMA n of NMF in a phase: spread evenly, so that a wave stalled on
             // a DMA issue still has MFMAs in the pipe
-            auto dma_after = [&](int n, int nmf, int ksx) {
+            auto dma_after = [&](int n, int nmf, int ksx, auto nt) {
 #pragma unroll
                 for (int q = n * LOADS / nmf; q < (n + 1) * LOADS / nmf; ++q)
-                    dma_ks(ksx, q);
+                    dma_ks(ksx, q, nt);
+            };
+            auto by_policy = [&](auto f) {
+                if constexpr (POL != W_BY_TILE)
+                    f(std::bool_constant<POL == W_STREAM>{});
+                else if (cur.nt)
+                    f(std::true_type{});
+                else
+                    f(std::false_type{});
             };
             if (!primed) {
                 if constexpr (CONSUME) {
                     if (cur_ready < SY().target)
                         wait_ready(mti_ctx(cur));
                 }
+                auto first = [&](auto nt) {
 #pragma unroll
-                for (int s0 = 0; s0 < GSTAGES; ++s0)
+                    for (int s0 = 0; s0 < GSTAGES; ++s0)
 #pragma unroll
-                    for (int q = 0; q < LOADS; ++q)
-                        dma_one(cur, min(s0, nk - 1), slot(s0), q);
+                        for (int q = 0; q < LOADS; ++q)
+                            dma_one(cur, min(s0, nk - 1), slot(s0), q, nt);
+                };
+                by_policy(first);
             }
             wait_vmcnt<LOADS *(GSTAGES - 1)>();  // k-step 0 has landed
             bar();
@@ -1139,15 +1209,6 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             const bool poll_next = chain;  // EAGER consumer: decided inside the k-loop
             if constexpr (EAGER_C)
                 chain = 0;
-            if constexpr (CONSUME && !EAGER) {
-                // the next tile's counter (bar() is a compiler memory barrier: the slot is read afresh), then
-                // the copy of the one after it into the slot this tile's counter occupied
-                if (chain)
-                    chain = __builtin_amdgcn_readfirstlane(rslot[(kt & 1) * 64]) >= SY().target;
-                const int t2 = seq(kt + 1);
-                if (t2 < total && w == 0)
-                    dma4_sc1(SY().ready + mti_of(t2), rslot + ((kt + 1) & 1) * 64);
-            }
             clear_acc();
             // end of a k-step: k-step ks+1 has landed for every wave and every wave has read k-step ks
             int edge = 0;
@@ -1222,7 +1283,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                 };
                 // MFMAs of the k-step held in (a, wr); A rows of k-step ks_next are read behind them and
                 // the DMA of k-step ks_next-1+STAGES is spread between them
-                auto mm = [&](const WRegs &wr, int ks_next, auto act) {
+                auto mm = [&](const WRegs &wr, int ks_next, auto act, auto nt) {
                     const int ks_dma = ks_next - 1 + GSTAGES;
 #pragma unroll
                     for (int i = 0; i < IF; ++i) {
@@ -1241,7 +1302,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                                 // in SwiGLU tiles a wave's columns j < JF/2 are gate rows, the rest up rows
                                 ps[j] = (SWIGLU && j >= JF / 2) ? sui : sgi;
                             }
-                            dma_after(i * JF + j, IF * JF, ks_dma);
+                            dma_after(i * JF + j, IF * JF, ks_dma, nt);
                             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
                             __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // 4 VALU
                             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // a DMA, where one follows
@@ -1254,25 +1315,27 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                 for (int i = 0; i < IF; ++i)
                     rd_a(i, 0);
                 rd_w(w0, 0);
-                auto kloop = [&](auto act) {
+                auto kloop = [&](auto act, auto nt) {
                     int ks = 0;
                     for (; ks + 1 < nk; ks += 2) {
                         step_edge();
                         rd_w(w1, ks + 1);
-                        mm(w0, ks + 1, act);
+                        mm(w0, ks + 1, act, nt);
                         step_edge();
                         rd_w(w0, ks + 2);
-                        mm(w1, ks + 2, act);
+                        mm(w1, ks + 2, act, nt);
                     }
                     if (ks < nk) {
                         step_edge();
-                        mm(w0, ks + 1, act);
+                        mm(w0, ks + 1, act, nt);
                     }
                 };
                 if (!spect && (TC::WAVES_M == 1 || cur.active))  // (one row-wave: a tile always has rows for it)
-                    kloop(std::true_type{});
-                else if constexpr (TC::WAVES_M > 1 || ROLE != SYNC_NONE)
-                    kloop(std::false_type{});
+                    by_policy([&](auto nt) { kloop(std::true_type{}, nt); });
+                else if constexpr (TC::WAVES_M > 1)
+                    by_policy([&](auto nt) { kloop(std::false_type{}, nt); });
+                else if constexpr (ROLE != SYNC_NONE)
+                    kloop(std::false_type{}, std::false_type{});  // spectators issue no DMA
 #pragma unroll
                 for (int j = 0; j < JF; ++j)  // the last row's pending results
 #pragma unroll
@@ -1297,13 +1360,13 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                         f.b[j] = *reinterpret_cast<const i32x4 *>(lb + swz(j * 16 + l16, ph * 4 + lg));
                 };
                 // MFMAs of one phase; with ks_dma >= 0 the DMA of that k-step is spread between them
-                auto mm = [&](const Regs &f, int ks_dma, auto act) {
+                auto mm = [&](const Regs &f, int ks_dma, auto act, auto nt) {
 #pragma unroll
                     for (int i = 0; i < IF; ++i)
 #pragma unroll
                         for (int j = 0; j < JF; ++j) {
                             if (ks_dma >= 0)
-                                dma_after(i * JF + j, IF * JF, ks_dma);
+                                dma_after(i * JF + j, IF * JF, ks_dma, nt);
                             if constexpr (!decltype(act)::value)
                                 ;
                             else if constexpr (INT8)
@@ -1318,26 +1381,48 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
                 };
                 Regs r0, r1;
                 rd(r0, 0, 0);
-                auto kloop = [&](auto act) {
+                auto kloop = [&](auto act, auto nt) {
                     for (int ks = 0; ks < nk; ++ks) {
                         rd(r1, ks, 1);
-                        mm(r0, -1, act);
+                        mm(r0, -1, act, nt);
                         step_edge();
                         rd(r0, ks + 1, 0);
-                        mm(r1, ks + GSTAGES, act);
+                        mm(r1, ks + GSTAGES, act, nt);
                     }
                 };
                 if (!spect && (TC::WAVES_M == 1 || cur.active))  // (one row-wave: a tile always has rows for it)
-                    kloop(std::true_type{});
-                else if constexpr (TC::WAVES_M > 1 || ROLE != SYNC_NONE)
-                    kloop(std::false_type{});
+                    by_policy([&](auto nt) { kloop(std::true_type{}, nt); });
+                else if constexpr (TC::WAVES_M > 1)
+                    by_policy([&](auto nt) { kloop(std::false_type{}, nt); });
+                else if constexpr (ROLE != SYNC_NONE)
+                    kloop(std::false_type{}, std::false_type{});  // spectators issue no DMA
             }
 
             // producer, primed tile: the previous tile's stores are counted now -- the k-loop's last edge left
             // at most LOADS (STAGES - 2) DMAs in flight in every wave, all issued after those stores
             signal();
             dequant_int8(cur);
-            if (!chain) {
+            if constexpr (DYNL) {
+                const int t = take();
+                wait_vmcnt<0>();  // the tail's reloads (and the ticket) have landed
+                tk = publish(t);
+                ntile = ticket_tile(tk);
+                has_next = ntile < total;
+                if (has_next) {
+                    setup(ntile, nxt);
+                    cur_ready = 0;
+                    if constexpr (CONSUME)
+                        cur_ready = spect ? 0 : poll(mti_ctx(nxt));
+                    if (can_chain && (!CONSUME || cur_ready >= SY().target)) {
+                        chain = 1;
+#pragma unroll
+                        for (int s0 = 0; s0 < GSTAGES; ++s0)
+#pragma unroll
+                            for (int q = 0; q < LOADS; ++q)
+                                dma_one(nxt, s0, slot(nk + s0), q, std::bool_constant<POL == W_STREAM>{});
+                    }
+                }
+            } else if (!chain) {
                 if constexpr (CONSUME) {
                     if (has_next && !gave_up && !spect)
                         cur_ready = poll(mti_ctx(nxt));  // answered while the ring drains
@@ -1361,6 +1446,7 @@ __device__ __forceinline__ void gmm_body(const GmmArgs &p, const GroupTables *gt
             bar();
             signal();
         }
+        return tk;
     }
 }
 
@@ -1387,17 +1473,18 @@ constexpr size_t G_LDS_BIG_BYTES =
     sizeof(GroupTables);
 static_assert(G_LDS_SMALL_BYTES <= 163840 && G_LDS_BIG_BYTES <= 163840, "LDS budget of a gfx950 workgroup");
 // the table scan's per-wave totals (before any ring use)
-static_assert(sizeof(int) * 4 * (GMAX_THREADS / 64) <= ring_bytes<32, 128>(), "table-scan scratch");
+static_assert(sizeof(int) * (G_NCLASS + 2) * (GMAX_THREADS / 64) <= ring_bytes<32, 128>(), "table-scan scratch");
 
-// Decode-sized segments: the 32-row tile (4 waves).
-template <int DT, int EPI> __global__ __launch_bounds__(256, 1) void gmm_kernel_small(GmmArgs p)
+// Decode-sized segments: the 32-row tile (4 waves).  Bounded to two waves per SIMD although the LDS allows one: with up
+// to 512 registers a wave the compiler keeps operands in accumulation registers and moves 24 to 64 of them per k-step.
+template <int DT, int EPI> __global__ __launch_bounds__(256, 2) void gmm_kernel_small(GmmArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     build_group_tables<Tile<32>::THREADS>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
-                                          ClassRanges{{0, 0, 0}, {0, 0, 0x7fffffff}});
-    gmm_body<DT, EPI, 32>(p, gt, -1, 0, 0, 1, -1, wv);
+                                          ClassRanges{{0, 0, 0, 0}, {0, 0, 0, 0x7fffffff}});
+    gmm_body<DT, EPI, CLS_32, SYNC_NONE, false, W_BY_TILE>(p, gt, -1, 0, 0, 1, wv);
 }
 
 // Prefill: 8 waves, 128- or 256-row tile picked per launch from the actual rows per touched
@@ -1408,14 +1495,12 @@ constexpr int G_HEAVY_ROWS = 384;
 // four of the block's waves: their tiles are a weight stream, and that tile's four-stage ring keeps half as
 // many weight bytes again in flight per CU as the 128-row tile's three stages (measured on config 4's fp8
 // GMM1: such a tile streams its 1.8 MB in 46-58 us against 51-65 us, the GEMM 186 vs 193 us; the int8 GEMM
-// measured 1-2% slower and keeps the 128-row tile).
+// measured 1-2% slower and keeps the 128-row tile).  One 32-row tile per expert: two of them would fetch its
+// weights twice.
 #ifndef CAM_GMM_SMALL_ROWS
-#define CAM_GMM_SMALL_ROWS 64
+#define CAM_GMM_SMALL_ROWS 33
 #endif
 constexpr int G_SMALL_ROWS = CAM_GMM_SMALL_ROWS;
-#ifndef CAM_GMM_RUN32
-#define CAM_GMM_RUN32 3
-#endif
 
 // Between two tile classes the block meets at an LDS-only barrier (lds_sync): both prefill loops have drained
 // their DMAs before the last epilogue, so only the ring's LDS reads must be complete (__syncthreads would also
@@ -1425,8 +1510,7 @@ constexpr int G_SMALL_ROWS = CAM_GMM_SMALL_ROWS;
 // sequence of each block continuing round-robin from the first class into the second, and (fp8, bf16) from
 // there into a third, the experts with fewer than G_SMALL_ROWS rows on 32-row tiles.  A layer whose
 // load is skewed (a few experts with a thousand rows, many with a handful) gets tall tiles where they
-// halve the operand traffic and short ones where a tall tile would multiply padding.  The light experts'
-// (at most three M-tiles each) weights are fetched nontemporally.
+// halve the operand traffic and short ones where a tall tile would multiply padding.
 // short reductions keep the 128-row tile: the 256-row tile's per-tile ring fill and drain would
 // not amortise over fewer than 16 k-steps (at 16, GMM2 of DeepSeek-V3's shapes: the M = 65536 fp8 GMM2
 // 1.71 vs 1.57 PFLOPS, int8 1.97 vs 1.67 POPS, config 4's fp8 GMM2 116 vs 122 us)
@@ -1434,128 +1518,164 @@ __host__ __device__ constexpr bool big_tall(int allow256, int K, int dt)
 {
     return allow256 && (int)((uint32_t)K * (dt == DT_BF16 ? 2 : 1) / GKB) >= CAM_GMM_MIN_NK256;
 }
-template <int DT> __device__ __forceinline__ ClassRanges big_ranges(bool tall)
+// heavy: the launch has experts for 256-row tiles; int8: the single 128-row tiles beside them are a class of their
+// own (fp8 and bf16 move their smallest experts to 32-row tiles instead, and one GEMM loop fewer in their kernels leaves
+// the 256-row loop more registers: 157 against 238 spilled scalars in the fp8 GMM1)
+template <int DT> __device__ __forceinline__ ClassRanges big_ranges(bool tall, bool heavy)
 {
     constexpr int SMALL = DT == DT_INT8 ? 1 : G_SMALL_ROWS;  // rows below: the 32-row tile class
-    return tall ? ClassRanges{{G_HEAVY_ROWS, SMALL, 1}, {0x7fffffff, G_HEAVY_ROWS, SMALL}}
-                : ClassRanges{{0, 0, 0}, {0, 0x7fffffff, 0}};
+    const int top = tall ? G_HEAVY_ROWS : 0x7fffffff, small = tall ? SMALL : 1;
+    const int multi = heavy && DT == DT_INT8 ? 129 : small;
+    return ClassRanges{{top, multi, small, 1}, {0x7fffffff, top, multi, small}};
 }
 
-// The 8-wave schedule of one GEMM over the tile classes of the launch's tables (gmm_kernel_big).  ROLE !=
-// SYNC_NONE (the chained kernel): the 32-row class keeps the block's other four waves as spectators instead of
-// ending them, since the block has more work after it.
-// bid: the block's id for the placement (blockIdx.x; a chained consumer passes its arrival order, so that the
-// blocks that finish GMM1 first take the positions with the most GMM2 work).
+// The 8-wave schedule of one GEMM over the tile classes of the launch's tables (gmm_kernel_big, gmm_chain_big): the
+// 256-row tiles first, then the light ones (128-row, then 32-row).  ROLE != SYNC_NONE (the chained kernel): the
+// 32-row class keeps the block's other four waves as spectators instead of ending them, since the block has more
+// work after it.
 template <int DT, int EPI, int ROLE>
-__device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables *gt, bool tall, int bid, int wv)
+__device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables *gt, int wv)
 {
-    const int pos = (gridDim.x & 7) ? bid : (bid & 7) * (int)(gridDim.x >> 3) + (bid >> 3);  // XCD-aware order
-    constexpr int SMALL = DT == DT_INT8 ? 1 : G_SMALL_ROWS;  // rows below: the 32-row tile class
+    const int G = gridDim.x, bid = blockIdx.x;
+    const int pos = (G & 7) ? bid : (bid & 7) * (G >> 3) + (bid >> 3);  // XCD-aware order
     constexpr bool KEEP = ROLE != SYNC_NONE;
-    if (!tall) {
-        gmm_body<DT, EPI, 128, false, ROLE>(p, gt, -1, 0, 0, 1, bid, wv);
-        return;
-    }
-    // light tiles worth about one heavy tile: a 256-row tile against 128-row tiles (2 for 1-byte operands, 1
-    // for bf16) or 32-row tiles (a plain one holds 128 W rows, a SwiGLU one 256: measured 35 and 105 us per
-    // heavy tile against 9 and 45-55 us per light one)
-    constexpr int run = DT == DT_BF16 ? 1 : 2;
-    constexpr int run32 = EPI == EPI_PLAIN ? 4 : CAM_GMM_RUN32;
-    // (uniform values read from LDS go to scalar registers at once: a VGPR holding one across the classes gets
-    // spilled, and its reload after a tile's k-loop makes the next k-loop wait for it at every iteration)
-    const int n_heavy = __builtin_amdgcn_readfirstlane(gt->tile_end[0][p.L - 1]);  // 256-row M-tiles (heavy)
-    const bool has_mid = __builtin_amdgcn_readfirstlane(gt->tile_end[1][p.L - 1]) > 0;
-    const bool has_small = __builtin_amdgcn_readfirstlane(gt->tile_end[2][p.L - 1]) > 0;
-    const int G = gridDim.x;
-    // 256-row tiles: heavy M-tiles x N-tiles
-    const int heavy_tiles = n_heavy * (EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / 256);
+    constexpr bool HAS32 = DT != DT_INT8;
+    // tiles of each class (uniform values read from LDS go to scalar registers at once: a VGPR holding one across
+    // the classes gets spilled, and its reload after a tile's k-loop makes the next k-loop wait for it at every
+    // iteration)
+    const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / 256, ntn32 = EPI != EPI_PLAIN ? ntn : p.N / small_bn(32, EPI);
+    const int n0 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_256>(p.L - 1)) * ntn;
+    const int n1 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_128M>(p.L - 1)) * ntn;
+    const int n2 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_128S>(p.L - 1)) * ntn;
+    const int n3 = HAS32 ? __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn32 : 0;
+    // Blocks that share n equal tiles in whole rounds: with R = ceil(n / G) rounds, only the first ceil(n / R) blocks
+    // (rounded up to whole XCDs) take tiles, R each at most, so a last partial round does not leave a few blocks
+    // streaming alone and a handful of tiles spreads over the XCDs.
+    auto blocks_for = [&](int n) {
+        const int rounds = max((n + G - 1) / G, 1);
+        return (G & 7) ? G : min(G, ((n + rounds - 1) / rounds + 7) / 8 * 8);
+    };
+    // this block's place among the first g blocks, XCD by XCD; far past every tile for the others
+    auto place = [&](int g) { return (G & 7) ? bid : bid < g ? (bid & 7) * (g >> 3) + (bid >> 3) : 0x3fffffff; };
+    // A chained GEMM's light tiles: one queue over the two classes, longest tiles first.  (Tile times differ by a
+    // factor of two with the load on the memory, so no static plan ends evenly: a layer of 22 touched experts, one of
+    // 2311 rows, ended its GMM1 between 66 and 303 us under round-robin, against 175 us of work per block.)
+    auto light_queue = [&](TileQueue q) {
+        if constexpr (ROLE != SYNC_NONE) {
+            q.end = n1;
+            if (n1 > 0) {
+                q.tk = gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, 0, 0, 0, 1, wv, q);
+                lds_sync();
+            }
+            q.base = q.end, q.end += n3;
+            if constexpr (HAS32) {
+                if (n3 > 0)
+                    gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, 0, 0, 0, 1, wv, q);
+            }
+        }
+    };
     if constexpr (ROLE == SYNC_CONSUME) {
         // Chained GMM2: the blocks reach it at different times (their GMM1 work differs), so the heavy tiles go
         // out through dynamic queues, one per XCD over that XCD's consecutive share (tiles sharing its L2), to
-        // whichever of its blocks is free; the light tiles follow round-robin by the blocks' arrival order.
-        if (heavy_tiles > 0) {
+        // whichever of its blocks is free; the light tiles follow from one queue.
+        if (n0 > 0) {
             const int nq = (G & 7) ? 1 : 8, x = nq == 1 ? 0 : (bid & 7);
-            const int hx = (heavy_tiles + nq - 1) / nq;
-            const int len = max(0, min(hx, heavy_tiles - x * hx));
-            gmm_body<DT, EPI, 256, false, ROLE>(p, gt, G_DYN, x * hx, len, chain_queue_index(p.M, p.L) + x, -1, wv);
+            const int hx = (n0 + nq - 1) / nq;
+            const int len = max(0, min(hx, n0 - x * hx));
+            gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, 0, 0, 0, 1, wv,
+                                             TileQueue{chain_queue_index(p.M, p.L) + x, 0, 0, len, x * hx, -1});
             lds_sync();
         }
-        if (has_mid)
-            gmm_body<DT, EPI, 128, true, ROLE>(p, gt, pos, 0, 0, 1, -1, wv);
-        if constexpr (SMALL > 1) {
-            if (has_small) {
-                lds_sync();
-                gmm_body<DT, EPI, 32, true, ROLE>(p, gt, pos, 0, 0, 1, -1, wv);
-            }
-        }
+        TileQueue q{chain_light_index(p.M, p.L, true), 0, 0, 0, 0, -1};
+        light_queue(q);
         return;
     }
-    if (heavy_tiles > 0 && heavy_tiles < G && (G & 7) == 0) {
+    // The heavy tiles leave some of the ge blocks at work free (with one heavy tile fewer than the others): nfree of
+    // them.  rank: this block's number among the free ones (is_free) or among the others, XCD by XCD.
+    int ge = G;
+    if (n0 == 0)
+        ge = ROLE == SYNC_PRODUCE && n1 + n2 + n3 >= G ? G : blocks_for(n1 + n2 + n3);
+    int nfree = ge, rank = place(ge);
+    bool is_free = rank < ge;
+    if (n0 > 0 && n0 < G && (G & 7) == 0) {
         // Fewer heavy tiles than blocks.  They are split evenly over the 8 XCDs (XCD x takes the run
         // [x hx, (x + 1) hx), consecutive tiles sharing that XCD's L2), so each XCD keeps some blocks free.
-        // The free blocks start on the light tiles at once, `run` (or `run32`) in a row each; the rest of
-        // the light tiles go round-robin over all blocks in launch order (every XCD in turn), reaching the
-        // heavy blocks as they finish.
         const int xcd = bid & 7, slot = bid >> 3, S = G >> 3;
-        const int hx = (heavy_tiles + 7) / 8;
-        auto heavy_in = [&](int x) { return max(0, min(hx, heavy_tiles - x * hx)); };
+        const int hx = (n0 + 7) / 8;
+        auto heavy_in = [&](int x) { return max(0, min(hx, n0 - x * hx)); };
         const int len = heavy_in(xcd);
         if (slot < len) {
-            gmm_body<DT, EPI, 256, false, ROLE>(p, gt, 0x3fffffff, xcd * hx + slot, (len - slot + S - 1) / S, S, -1, wv);
+            gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, 0x3fffffff, xcd * hx + slot, (len - slot + S - 1) / S, S, wv);
             lds_sync();  // every wave is done with the first class's ring
         }
-        int free_before = 0, free_all = 0;
+        int free_before = 0, busy_before = 0;
+        nfree = 0;
         for (int x = 0; x < 8; ++x) {
-            const int fx = max(0, S - heavy_in(x));
-            free_before += x < xcd ? fx : 0;
-            free_all += fx;
+            const int h = heavy_in(x);
+            free_before += x < xcd ? S - h : 0;
+            busy_before += x < xcd ? h : 0;
+            nfree += S - h;
         }
-        const bool is_free = slot >= len;
-        const int fpos = free_before + slot - len;  // the block's rank among the free blocks
-        if (has_mid)
-            gmm_body<DT, EPI, 128, true, ROLE>(p, gt, run * free_all + bid, is_free ? fpos * run : 0, is_free ? run : 0, 1, -1, wv);
-        if constexpr (SMALL > 1) {
-            if (has_small) {
-                lds_sync();
-                if (!KEEP && wv >= Tile<32>::NWAVES)
-                    return;  // the 32-row tile's four waves go on (a barrier only counts the waves still running)
-                gmm_body<DT, EPI, 32, true, ROLE>(p, gt, run32 * free_all + bid, is_free ? fpos * run32 : 0, is_free ? run32 : 0, 1, -1, wv);
-            }
-        }
+        is_free = slot >= len;
+        rank = is_free ? free_before + slot - len : busy_before + slot;
+    } else if (n0 > 0) {
+        // At least as many heavy tiles as blocks: round-robin, so the first n0 % G blocks run one more than the rest
+        gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, pos, 0, 0, 1, wv);
+        lds_sync();
+        const int r = n0 % G;
+        nfree = G - r;
+        is_free = pos >= r;
+        rank = is_free ? pos - r : pos;
+    }
+    if constexpr (ROLE == SYNC_PRODUCE) {
+        // the light tiles through one queue; the free blocks start at their own place in it
+        TileQueue q{chain_light_index(p.M, p.L, false), nfree, 0, 0, 0, is_free ? rank : -1};
+        light_queue(q);
         return;
     }
-    if (n_heavy == 0) {  // one class after another, each balanced over the blocks
-        if (has_mid)
-            gmm_body<DT, EPI, 128, true, ROLE>(p, gt, -1, 0, 0, 1, bid, wv);
-        if constexpr (SMALL > 1) {
-            if (has_small) {
-                lds_sync();
-                if (!KEEP && wv >= Tile<32>::NWAVES)
-                    return;
-                gmm_body<DT, EPI, 32, true, ROLE>(p, gt, -1, 0, 0, 1, bid, wv);
-            }
+    // Static plan: layer by layer, each layer one light tile for every block of the group (the free blocks, the others)
+    // that then ends first, counted in 20ths of a heavy tile's time.  A light tile's time against a heavy one's: 14/20 for
+    // a 128-row tile (measured 73 against 105 us in GMM1, 24 against 34 us in GMM2; int8 66 against 95 us), 11/20 and
+    // 5/20 for a 32-row tile with and without SwiGLU.  Within a group the tiles go round-robin, the sequence going on
+    // from class to class.
+    const int nbusy = ge - nfree, ng = is_free ? nfree : nbusy;
+    int busy_end = 20, free_end = 0, at = 0;
+    auto light = [&](int n, int cost, int &rs, int &rn) {
+        int nf = 0, nb = 0;  // tiles of the free blocks, of the others
+        while (nf + nb < n) {
+            const bool f = nfree > 0 && (nbusy == 0 || free_end <= busy_end);
+            const int layer = min(n - nf - nb, f ? nfree : nbusy);
+            nf += f ? layer : 0;
+            nb += f ? 0 : layer;
+            free_end += f ? cost : 0;
+            busy_end += f ? 0 : cost;
         }
-        return;
+        const int mine = is_free ? nf : nb, r = rank < ng ? (rank - at + ng) % ng : 0x3fffffff;
+        // (divisions leave their results in vector registers: scalar ones, as above)
+        rs = __builtin_amdgcn_readfirstlane((is_free ? 0 : nf) + r);
+        rn = __builtin_amdgcn_readfirstlane(max(0, (mine - r + ng - 1) / max(ng, 1)));
+        at = __builtin_amdgcn_readfirstlane((at + mine) % max(ng, 1));
+        free_end = __builtin_amdgcn_readfirstlane(free_end);
+        busy_end = __builtin_amdgcn_readfirstlane(busy_end);
+    };
+    int rs, rn;
+    if (n1 > 0) {
+        light(n1, 14, rs, rn);
+        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
+        lds_sync();
     }
-    // At least as many heavy tiles as blocks: they go round-robin over the blocks, so the first
-    // heavy_tiles % G blocks run one more of them than the rest.  Those others (the free blocks) start the
-    // light tiles with a run of about one heavy tile's worth each; the rest of the light tiles go
-    // round-robin over all blocks (measured on config 4's GMM2, 364 heavy tiles on 256 blocks: the light
-    // tiles' round-robin then no longer lands on blocks still busy with their second heavy tile).
-    gmm_body<DT, EPI, 256, false, ROLE>(p, gt, pos, 0, 0, 1, -1, wv);
-    lds_sync();  // every wave is done with the first class's ring
-    const int r = heavy_tiles % G;
-    const int nfree = r > 0 ? G - r : 0;
-    const bool is_free = nfree > 0 && pos >= r;
-    const int fpos = pos - r;
-    if (has_mid)
-        gmm_body<DT, EPI, 128, true, ROLE>(p, gt, run * nfree + pos, is_free ? fpos * run : 0, is_free ? run : 0, 1, -1, wv);
-    if constexpr (SMALL > 1) {
-        if (has_small) {
-            lds_sync();
+    if constexpr (DT == DT_INT8) {
+        if (n2 > 0) {
+            light(n2, 14, rs, rn);
+            gmm_body<DT, EPI, CLS_128S, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
+        }
+    }
+    if constexpr (HAS32) {
+        if (n3 > 0) {
+            light(n3, EPI == EPI_PLAIN ? 5 : 11, rs, rn);
             if (!KEEP && wv >= Tile<32>::NWAVES)
-                return;
-            gmm_body<DT, EPI, 32, true, ROLE>(p, gt, run32 * nfree + pos, is_free ? fpos * run32 : 0, is_free ? run32 : 0, 1, -1, wv);
+                return;  // the 32-row tile's four waves go on (a barrier only counts the waves still running)
+            gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
         }
     }
 }
@@ -1567,8 +1687,9 @@ template <int DT, int EPI> __global__ __launch_bounds__(512, 1) void gmm_kernel_
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const bool tall = big_tall(p.allow256, p.K, DT);
     // every class's expert table, from one read of the counts
-    build_group_tables<GMAX_THREADS>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), big_ranges<DT>(tall));
-    big_schedule<DT, EPI, SYNC_NONE>(p, gt, tall, (int)blockIdx.x, wv);
+    build_group_tables<GMAX_THREADS>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
+                                     big_ranges<DT>(tall, false), tall ? G_HEAVY_ROWS : 0, big_ranges<DT>(tall, true));
+    big_schedule<DT, EPI, SYNC_NONE>(p, gt, wv);
 }
 
 // Chained GMM1 + SwiGLU -> GMM2 (launch_gmm_chain): one table build, every block's GMM1 tiles (producing), then
@@ -1576,23 +1697,6 @@ template <int DT, int EPI> __global__ __launch_bounds__(512, 1) void gmm_kernel_
 // tiles before its first wait, so with every block resident each wait ends; a wait that outlasts the bound
 // gives up instead (and the host reads the sync status).  The grid is one block per CU, the blocks' LDS keeps
 // them to one per CU.
-// The block's arrival order at the GMM1 -> GMM2 boundary, as a block id: its rank among the blocks of its XCD
-// (one counter per XCD, after the M-tile counters) in place of blockIdx.x >> 3.  The consumer phase places its
-// tiles by it: the blocks that finish GMM1 first take the positions that hold the most GMM2 work.
-__device__ __forceinline__ int arrival_bid(int M, int L, uint8_t *smem, int wv)
-{
-    int *slot = reinterpret_cast<int *>(smem);  // the ring is idle between the phases
-    const int xcd = blockIdx.x & 7;
-    if (wv == 0 && lane_id() == 0) {
-        int *ctr = chain_params()->sy.ready + chain_arrival_index(M, L) + xcd;
-        *slot = __hip_atomic_fetch_add(gptr(ctr), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    const int r = *slot;
-    __syncthreads();  // (the slot is ring memory again)
-    return (gridDim.x & 7) ? (int)blockIdx.x : r * 8 + xcd;
-}
-
 template <int DT, int EPI1> __global__ __launch_bounds__(512, 1) void gmm_chain_big(ChainParams cp)
 {
     (void)cp;  // read through chain_params()
@@ -1604,15 +1708,14 @@ template <int DT, int EPI1> __global__ __launch_bounds__(512, 1) void gmm_chain_
         const GmmArgs p1 = chain_params()->g1;
         tall = big_tall(p1.allow256, p1.K, DT);  // the host checked that GMM2 makes the same choice
         build_group_tables<GMAX_THREADS>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                         big_ranges<DT>(tall));
-        big_schedule<DT, EPI1, SYNC_PRODUCE>(p1, gt, tall, (int)blockIdx.x, wv);
+                                         big_ranges<DT>(tall, false));
+        big_schedule<DT, EPI1, SYNC_PRODUCE>(p1, gt, wv);
     }
     lds_sync();  // every wave is done with GMM1's last ring
     const GmmArgs p2 = chain_params()->g2;
-    const int bid = arrival_bid(p2.M, p2.L, smem, wv);
-    big_schedule<DT, EPI_PLAIN, SYNC_CONSUME>(p2, gt, tall, bid, wv);
+    big_schedule<DT, EPI_PLAIN, SYNC_CONSUME>(p2, gt, wv);
 }
-template <int DT, int EPI1> __global__ __launch_bounds__(256, 1) void gmm_chain_small(ChainParams cp)
+template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_small(ChainParams cp)
 {
     (void)cp;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -1627,18 +1730,22 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 1) void gmm_chain_
     {
         const GmmArgs p1 = chain_params()->g1;
         build_group_tables<Tile<32>::THREADS>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                              ClassRanges{{0, 0, 0}, {0, 0, 0x7fffffff}});
-        t1 = gt->tile_end[2][p1.L - 1] * (p1.N / 2 / 128);
-        gmm_body<DT, EPI1, 32, true, SYNC_PRODUCE, true>(p1, gt, pos, 0, 0, 1, -1, wv);
+                                              ClassRanges{{0, 0, 0, 0}, {0, 0, 0, 0x7fffffff}});
+        t1 = gt->template end<CLS_32>(p1.L - 1) * (p1.N / 2 / 128);
+        gmm_body<DT, EPI1, CLS_32, SYNC_PRODUCE, true, W_BY_TILE>(p1, gt, pos, 0, 0, 1, wv);
     }
     lds_sync();
     const GmmArgs p2 = chain_params()->g2;
     const int r1 = t1 % G, nfree = r1 ? G - r1 : 0;
     const bool is_free = nfree > 0 && pos >= r1;
     constexpr int BN2 = small_bn(32, EPI_PLAIN);
-    const int R = max(1, (GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K));
-    gmm_body<DT, EPI_PLAIN, 32, true, SYNC_CONSUME, true>(p2, gt, R * nfree + pos, is_free ? (pos - r1) * R : 0,
-                                                          is_free ? R : 0, 1, -1, wv);
+    // (never more than spreads GMM2's tiles over the free blocks: with few tiles a run would leave most of them idle;
+    // one token through 2 of 8 bf16 experts, H = 1024: 16 GMM2 tiles on 16 blocks instead of 4)
+    const int t2 = gt->template end<CLS_32>(p2.L - 1) * (p2.N / BN2);
+    const int R = max(1, min((GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K),
+                             nfree ? (t2 + nfree - 1) / nfree : 1));
+    gmm_body<DT, EPI_PLAIN, CLS_32, SYNC_CONSUME, true, W_BY_TILE>(p2, gt, R * nfree + pos, is_free ? (pos - r1) * R : 0,
+                                                          is_free ? R : 0, 1, wv);
 }
 
 // Per-device launch state: the CU count and whether a kernel's dynamic-LDS limit has been raised.
@@ -1737,7 +1844,7 @@ hipError_t launch_gmm(const GmmArgs &a, int dt, int epi, hipStream_t s)
 #ifndef CAM_GMM_CHAIN_BIG
 #define CAM_GMM_CHAIN_BIG 1  // the prefill-sized chained kernel (8 waves, all tile classes)
 #endif
-int gmm_chain_counters(int M, int L) { return chain_queue_index(M, L) + 8; }
+int gmm_chain_counters(int M, int L) { return chain_light_index(M, L, true) + 1; }
 
 static bool chain_small(const GmmArgs &g) { return g.M <= 48 * g.L; }
 
