@@ -34,10 +34,12 @@ def test_chained_prefill_tiles_at_class_edges(lib, dt, case):  # noqa: F811
     assert lib.sync_status() == 0
 
 
-@pytest.mark.parametrize("counts", [[1, 0, 1, 0, 0, 0, 0, 0], [0, 3], [33, 1, 32, 40], [1] * 40])
+@pytest.mark.parametrize("counts", [[1, 0, 1, 0, 0, 0, 0, 0], [0, 3], [33, 1, 32, 40], [1] * 40, [64, 65, 31] * 8 + [0] * 8,
+                                    [40] * 48])
 @pytest.mark.parametrize("dt", [DT_FP8, DT_BF16])
-def test_chained_decode_few_tiles(lib, dt, counts):  # noqa: F811
-    # fewer GMM2 tiles than blocks without GMM1 work: they spread over the free blocks
+def test_chained_decode_tiles(lib, dt, counts):  # noqa: F811
+    # fewer GMM2 tiles than blocks without GMM1 work (they spread over the free blocks); 32- and 64-row tiles in one
+    # launch, one class alone, and a run of GMM2 tiles across the two
     print(f"chained decode counts={counts} dt={dt}", flush=True)
     c = Case(counts, 1024, 512, dt, 70)
     c.run_pair(lib)

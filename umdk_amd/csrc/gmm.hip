@@ -76,8 +76,10 @@ constexpr int G_MAX_L = 512;
 //   BM = 128: 8 waves, 2 x 4 of 64 x 64, 3-stage ring;
 //   BM = 32:  4 waves, 1 x 4 of 32 x 64, 4-stage ring (decode: a handful of rows per expert, the k-loop
 //             is a weight stream and the extra stage keeps more of it in flight);
-//   BM = 32, BN = 128: 4 waves of 32 x 32, 6-stage ring (the same bytes in flight) -- the decode GEMM
-//             without SwiGLU, whose tiles then divide evenly over the CUs.
+//   BM = 64:  4 waves, 1 x 4 of 64 x 64, 3-stage ring (a decode batch with more rows than that on an expert:
+//             its weights pass once where two 32-row tiles fetch them twice);
+//   BM = 32 or 64, BN = 128: 4 waves of 32 columns, 6-stage ring (the same bytes in flight) -- the decode
+//             GEMM without SwiGLU, whose tiles then divide evenly over the CUs.
 template <int BM_, int BN_ = GBN> struct Tile {
     static constexpr int BM = BM_, BN = BN_;
     static constexpr int NWAVES = BM >= 128 ? 8 : 4;
@@ -86,7 +88,7 @@ template <int BM_, int BN_ = GBN> struct Tile {
     static constexpr int WAVES_N = NWAVES / WAVES_M;
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // wave tile
     static constexpr int IF = WM / 16, JF = WN / 16;              // MFMA fragments per wave
-    static constexpr int STAGES = BM >= 256 ? 2 : BM >= 128 ? 3 : BN >= 256 ? 4 : 6;
+    static constexpr int STAGES = BM >= 256 ? 2 : BM >= 128 ? 3 : BN < 256 ? 6 : BM >= 64 ? 3 : 4;
     static constexpr int A_BYTES = BM * GKB;
     static constexpr int B_BYTES = BN * GKB;
     static constexpr int S_ROWS = WM > 64 ? WM : 64;  // activation-scale rows a wave DMAs (64 per instruction)
@@ -102,27 +104,27 @@ template <int BM_, int BN_ = GBN> struct Tile {
 #ifndef CAM_GMM_SMALL_PLAIN_BN
 #define CAM_GMM_SMALL_PLAIN_BN 128
 #endif
-constexpr int small_bn(int bm, int epi) { return bm == 32 && epi == 0 ? CAM_GMM_SMALL_PLAIN_BN : GBN; }
+constexpr int small_bn(int bm, int epi) { return bm <= 64 && epi == 0 ? CAM_GMM_SMALL_PLAIN_BN : GBN; }
 
 // Tile classes: 256-row tiles, 128-row tiles of experts with several of them, 128-row tiles of experts with one,
-// 32-row tiles.  The two 128-row classes differ in how they fetch their weights (see W_CACHED and W_STREAM).
-enum TileClass { CLS_256 = 0, CLS_128M = 1, CLS_128S = 2, CLS_32 = 3 };
+// 32-row tiles; and in the 4-wave kernels, in the place of CLS_128M, 64-row tiles.  The two 128-row classes differ in
+// how they fetch their weights (see W_CACHED and W_STREAM).
+enum TileClass { CLS_256 = 0, CLS_128M = 1, CLS_128S = 2, CLS_32 = 3, CLS_64 = 4 };
 constexpr int G_NCLASS = 4;
-constexpr int class_bm(int cls) { return cls == CLS_256 ? 256 : cls == CLS_32 ? 32 : 128; }
+constexpr int class_bm(int cls) { return cls == CLS_256 ? 256 : cls == CLS_32 ? 32 : cls == CLS_64 ? 64 : 128; }
 
 // Expert tables of a launch, built once at kernel start: per tile class the inclusive prefix of M-tiles per
 // expert, and the inclusive prefix of rows per expert (the exclusive prefix of expert e is entry e-1, or 0 for
 // e = 0; no entry for it keeps the tables within the LDS budget).  The last two classes share a word: at most one
-// tile per expert in CLS_128S (<= 512), and CLS_32 only ever takes experts of fewer than G_SMALL_ROWS rows or a
-// launch of at most 48 rows per expert (<= 1280 tiles).
+// tile per expert in either (<= 512), or few tiles in all (see small_ranges).
 struct GroupTables {
     int tile_end[G_NCLASS - 2][G_MAX_L];
     uint32_t tile_end_s[G_MAX_L];  // CLS_128S << 16 | CLS_32
     int row_end[G_MAX_L];
     template <int CLS> __device__ __forceinline__ int end(int e) const
     {
-        if constexpr (CLS < CLS_128S)
-            return tile_end[CLS][e];
+        if constexpr (CLS < CLS_128S || CLS == CLS_64)
+            return tile_end[CLS == CLS_64 ? CLS_128M : CLS][e];
         else
             return CLS == CLS_128S ? (int)(tile_end_s[e] >> 16) : (int)(tile_end_s[e] & 0xffffu);
     }
@@ -212,12 +214,14 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // the counts.  Only experts with a row count in a class's [lo, hi) get tiles of that class (a launch may
 // split the experts between tile heights); the row offsets count every expert (they locate segments in
 // dispatch order).
-template <int GTHREADS>
+template <int GTHREADS, bool FOUR_WAVES = false>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
-                                   ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{})
+                                   ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{},
+                                   int few_tiles = 0)
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
-    constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(1), class_bm(2), class_bm(3)};
+    constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(FOUR_WAVES ? CLS_64 : CLS_128M),
+                                   FOUR_WAVES ? 32 : class_bm(2), class_bm(3)};
     const int tid = threadIdx.x;
     const int per = (L + GTHREADS - 1) / GTHREADS;
     constexpr int NWV = GTHREADS / 64;
@@ -280,10 +284,25 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
             ex += v < wv ? scratch[k * NWV + v] : 0;
         run[k] = ex;
     }
+    bool few = false;
+    if constexpr (FOUR_WAVES) {  // slot 2 counts the M-tiles with 32-row tiles throughout (small_ranges)
+        int all32 = 0;
+#pragma unroll
+        for (int v = 0; v < NWV; ++v)
+            all32 += scratch[2 * NWV + v];
+        few = all32 <= few_tiles;
+    }
     for (int q = 0; q < per; ++q) {
         const int e = tid * per + q;
         if (e < L) {
             add((int)group_list[e], run);
+            if constexpr (FOUR_WAVES) {
+                gt.tile_end[CLS_256][e] = 0;
+                gt.tile_end[CLS_128M][e] = few ? 0 : run[CLS_128M];
+                gt.tile_end_s[e] = (uint32_t)(few ? run[2] : run[CLS_32]);
+                gt.row_end[e] = run[G_NCLASS];
+                continue;
+            }
             gt.tile_end[CLS_256][e] = run[CLS_256];
             gt.tile_end[CLS_128M][e] = run[CLS_128M];
             gt.tile_end_s[e] = (uint32_t)run[CLS_128S] << 16 | (uint32_t)run[CLS_32];
@@ -301,12 +320,14 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * GKB + ((ch
 // the lane's index in its wave, from mbcnt (no work-item id register)
 __device__ __forceinline__ int lane_id() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
-// the same, recomputed where it stands: what a tile switch derives from the lane is then not kept in registers through
-// the k-loop (which spills it, each reload waiting for every store of the epilogue before it)
-__device__ __forceinline__ int lane_here()
+// the same, recomputed where it stands (FRESH): what a tile switch derives from the lane is then not kept in registers
+// through the k-loop, which in the fp8 kernels spills it, each reload waiting for every store of the epilogue
+// before it.  The other kernels have the registers to keep it.
+template <bool FRESH> __device__ __forceinline__ int lane_here()
 {
     int l = lane_id();
-    asm volatile("" : "+v"(l));
+    if constexpr (FRESH)
+        asm volatile("" : "+v"(l));
     return l;
 }
 
@@ -391,9 +412,8 @@ __device__ __forceinline__ void lds_sync()
     bar();
 }
 
-// Tiles of the experts with a row count in [lo, hi); this block takes tiles first, first + G, ...
-// (first == -1: balanced placement, see below; G_DYN: a dynamic queue), preceded by a run of rn tiles rs, rs + rstride, ... (an
-// increasing sequence: the first index past the class's tiles ends it).
+// The tiles of one class: this block takes a run of rn tiles rs, rs + rstride, ..., then tiles first, first + G, ...
+// (an increasing sequence: the first index past the class's tiles ends it), or tickets of a queue.
 // ROLE (chained launches only): SYNC_PRODUCE tiles store h agent-coherently and count each finished tile in
 // sy.ready; SYNC_CONSUME tiles start their DMAs only once sy.ready of their M-tile has reached sy.target.  Waves
 // beyond the tile's own (a 32-row class run by an 8-wave block) are spectators: they issue no DMA, MFMA or store
@@ -418,6 +438,7 @@ struct TileQueue {
 // without heavy experts cached weights are as fast with many tiles (160 against 158 us for 48 experts of 100 rows) and
 // faster with few (54 against 60 us for one expert of 128 rows, N = 4096, K = 7168).
 enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
+constexpr int policy64(int dt) { return dt == DT_FP8 ? W_STREAM : W_BY_TILE; }  // (fp8: no registers for two loops)
 constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? W_STREAM : W_CACHED; }
 
 template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS)>
@@ -438,6 +459,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     auto tile_prefix = [&](int e) { return e > 0 ? tile_end(e - 1) : 0; };
     auto row_off = [&](int e) { return e > 0 ? gtab->row_end[e - 1] : 0; };
 
+    constexpr bool FRESH = DT == DT_FP8;
     const int lane = lane_id();
     const int w = wv >= 0 ? wv : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const bool first_thread = w == 0 && lane == 0;
@@ -448,11 +470,12 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     // M-tiles of the classes before this one (the readiness counters' index base), read when needed
     auto cls_base = [&]() {
         int b = 0;
-        if constexpr (CLS > CLS_256)
+        constexpr int SLOT = CLS == CLS_64 ? CLS_128M : CLS;
+        if constexpr (SLOT > CLS_256)
             b += gtab->template end<CLS_256>(p.L - 1);
-        if constexpr (CLS > CLS_128M)
+        if constexpr (SLOT > CLS_128M)
             b += gtab->template end<CLS_128M>(p.L - 1);
-        if constexpr (CLS > CLS_128S)
+        if constexpr (SLOT > CLS_128S)
             b += gtab->template end<CLS_128S>(p.L - 1);
         return __builtin_amdgcn_readfirstlane(b);
     };
@@ -467,26 +490,13 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     const int ntn = SWIGLU ? half_n / 128 : p.N / TBN;
     const int total = __builtin_amdgcn_readfirstlane(tile_prefix(p.L)) * ntn;
 
-    // first == -1: this launch has one tile class, so balance it: with R = ceil(total / grid) rounds, only
-    // the first ceil(total / R) blocks (rounded up to whole XCDs) take tiles, R each at most.  A weight
-    // stream is bound by aggregate HBM bandwidth, which that many CUs still saturate, and no CU is left
-    // streaming a final partial round alone.  Otherwise the caller's position and the full grid stride.
-    int G = gridDim.x, logical = first;
+    const int G = gridDim.x, logical = first;
     // tiles from the queue tq, in the 8-wave chained kernel: the consumer's heavy tiles (a queue per XCD) and the
     // light tiles of both GEMMs
     constexpr bool dyn = CONSUME && BM >= 256;
     constexpr bool DYNL = ROLE != SYNC_NONE && BM < 256 && !EAGER;
     int tk = tq.tk;
     auto ticket_tile = [&](int t) { return t < tq.end ? tq.first + t - tq.base : 0x7fffffff; };
-    if (first == -1) {
-        const int b = blockIdx.x;
-        const int rounds = max((total + G - 1) / G, 1);
-        const int g_eff = min(G, ((total + rounds - 1) / rounds + 7) / 8 * 8);
-        if (b >= g_eff)
-            return tk;
-        G = g_eff;
-        logical = (b & 7) * (G >> 3) + (b >> 3);
-    }
     // the block's k-th tile: the run, then the strided sequence
     auto seq = [&](int k) { return k < rn ? rs + k * rstride : logical + (k - rn) * G; };
 
@@ -504,7 +514,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         int nt;        // the expert's only M-tile (W_BY_TILE)
     };
     auto setup = [&](int tile, Ctx &c) {
-        const int lane = lane_here(), band_row = lane >> 3;
+        const int lane = lane_here<FRESH>(), band_row = lane >> 3;
         auto chunk_off = [&](int r) { return (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4); };
         int lo = 0, hi = p.L - 1;
         while (lo < hi) {  // last e with tile_prefix[e]*ntn <= tile
@@ -645,7 +655,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
             return;
         }
         const int row0 = c.row0, seg1 = c.seg1, n0 = c.n0;
-        const int lid = lane_here(), l16 = lid & 15, lg = lid >> 4;
+        const int lid = lane_here<FRESH>(), l16 = lid & 15, lg = lid >> 4;
         if constexpr (EPI == EPI_PLAIN) {
 #pragma unroll
             for (int i = 0; i < IF; ++i) {
@@ -778,7 +788,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     // v = ((float)acc * w_scale[n]) * x_scale[m]  (block_epilogue_per_token_dequant*.h)
     auto dequant_int8 = [&](const Ctx &cur) {
         if constexpr (INT8) {
-            const int lid = lane_here(), l16 = lid & 15, lg = lid >> 4;
+            const int lid = lane_here<FRESH>(), l16 = lid & 15, lg = lid >> 4;
             const float *wsr = cur.wsb;
 #pragma unroll
             for (int j = 0; j < JF; ++j) {
@@ -1458,6 +1468,22 @@ __device__ __forceinline__ int xcd_position()
     return (G & 7) ? (int)blockIdx.x : (int)((blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3));
 }
 
+// Blocks that share n equal tiles in whole rounds: with R = ceil(n / G) rounds, only the first ceil(n / R) blocks
+// (rounded up to whole XCDs) take tiles, R each at most, so a last partial round does not leave a few blocks streaming
+// alone and a handful of tiles spreads over the XCDs.
+__device__ __forceinline__ int blocks_for(int n)
+{
+    const int G = gridDim.x, rounds = max((n + G - 1) / G, 1);
+    return __builtin_amdgcn_readfirstlane((G & 7) ? G : min(G, ((n + rounds - 1) / rounds + 7) / 8 * 8));
+}
+// this block's place among the first g blocks, XCD by XCD; far past every tile for the others
+constexpr int G_NOWHERE = 0x3fffffff;
+__device__ __forceinline__ int place_among(int g)
+{
+    const int b = blockIdx.x;
+    return (gridDim.x & 7) ? b : b < g ? (b & 7) * (g >> 3) + (b >> 3) : G_NOWHERE;
+}
+
 // LDS of a launch: a class's ring of stages, then that class's epilogue exchange area; the expert tables
 // sit at the end of the launch's LDS (the same place for every class of a launch).
 template <int BM, int BN = GBN> constexpr size_t ring_bytes() { return Tile<BM, BN>::STAGES * Tile<BM, BN>::STAGE_BYTES; }
@@ -1467,7 +1493,8 @@ template <int BM, int BN = GBN> constexpr size_t exchange_bytes()
 }
 template <int BM, int BN = GBN> constexpr size_t class_bytes() { return ring_bytes<BM, BN>() + exchange_bytes<BM, BN>(); }
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
-constexpr size_t G_LDS_SMALL_BYTES = cmax(class_bytes<32, GBN>(), class_bytes<32, 128>()) + sizeof(GroupTables);
+constexpr size_t G_LDS_SMALL_BYTES = cmax(cmax(class_bytes<32, GBN>(), class_bytes<32, 128>()),
+                                          cmax(class_bytes<64, GBN>(), class_bytes<64, 128>())) + sizeof(GroupTables);
 constexpr size_t G_LDS_BIG_BYTES =
     cmax(cmax(class_bytes<256>(), class_bytes<128>()), cmax(class_bytes<32, GBN>(), class_bytes<32, 128>())) +
     sizeof(GroupTables);
@@ -1475,16 +1502,37 @@ static_assert(G_LDS_SMALL_BYTES <= 163840 && G_LDS_BIG_BYTES <= 163840, "LDS bud
 // the table scan's per-wave totals (before any ring use)
 static_assert(sizeof(int) * (G_NCLASS + 2) * (GMAX_THREADS / 64) <= ring_bytes<32, 128>(), "table-scan scratch");
 
-// Decode-sized segments: the 32-row tile (4 waves).  Bounded to two waves per SIMD although the LDS allows one: with up
-// to 512 registers a wave the compiler keeps operands in accumulation registers and moves 24 to 64 of them per k-step.
-template <int DT, int EPI> __global__ __launch_bounds__(256, 2) void gmm_kernel_small(GmmArgs p)
+// Decode-sized segments (4 waves): 32-row tiles, and 64-row tiles for the experts of more rows (64 bf16 experts of 37
+// rows on average, H = 2048, I = 1408: the decode step 245 us against 282 us with two 32-row tiles, each streaming the
+// expert's weights).  fp8 and bf16 are bounded to two waves per SIMD although the LDS allows one: with up to
+// 512 registers a wave the compiler keeps operands in accumulation registers and moves 24 to 64 of them per k-step (the
+// int8 GMM2 alone measured faster that way, 76 against 78 us).
+// With no more 32-row tiles than blocks they all run at once, and two of them end before one 64-row tile does (32 fp8
+// experts of 15 rows, K = 5888, two N-tiles each: GMM1 and GMM2 75 us against 78 us): 32-row tiles throughout then.
+constexpr int G_ROWS32 = 32;
+__device__ __forceinline__ ClassRanges small_ranges()
+{
+    return ClassRanges{{0, G_ROWS32 + 1, 1, 1}, {0, 0x7fffffff, 0x7fffffff, G_ROWS32 + 1}};
+}
+template <int DT, int EPI> __global__ __launch_bounds__(256, DT == DT_INT8 ? 1 : 2) void gmm_kernel_small(GmmArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    build_group_tables<Tile<32>::THREADS>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
-                                          ClassRanges{{0, 0, 0, 0}, {0, 0, 0, 0x7fffffff}});
-    gmm_body<DT, EPI, CLS_32, SYNC_NONE, false, W_BY_TILE>(p, gt, -1, 0, 0, 1, wv);
+    const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / small_bn(32, EPI);
+    build_group_tables<Tile<32>::THREADS, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(), 0,
+                                                ClassRanges{}, (int)gridDim.x / ntn);
+    const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p.L - 1)) * ntn;
+    const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn;
+    // one round-robin sequence over both classes (a tile of either streams the same weight bytes)
+    const int ge = blocks_for(n64 + n32), rank = place_among(ge);
+    auto rounds = [&](int r, int n) { return __builtin_amdgcn_readfirstlane(r < ge ? (n - r + ge - 1) / ge : 0); };
+    if (n64 > 0) {
+        gmm_body<DT, EPI, CLS_64, SYNC_NONE, false, policy64(DT)>(p, gt, G_NOWHERE, rank, rounds(rank, n64), ge, wv);
+        lds_sync();
+    }
+    const int r32 = __builtin_amdgcn_readfirstlane(rank < ge ? (rank + ge - n64 % ge) % ge : G_NOWHERE);
+    gmm_body<DT, EPI, CLS_32>(p, gt, G_NOWHERE, r32, rounds(r32, n32), ge, wv);
 }
 
 // Prefill: 8 waves, 128- or 256-row tile picked per launch from the actual rows per touched
@@ -1548,15 +1596,6 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     const int n1 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_128M>(p.L - 1)) * ntn;
     const int n2 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_128S>(p.L - 1)) * ntn;
     const int n3 = HAS32 ? __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn32 : 0;
-    // Blocks that share n equal tiles in whole rounds: with R = ceil(n / G) rounds, only the first ceil(n / R) blocks
-    // (rounded up to whole XCDs) take tiles, R each at most, so a last partial round does not leave a few blocks
-    // streaming alone and a handful of tiles spreads over the XCDs.
-    auto blocks_for = [&](int n) {
-        const int rounds = max((n + G - 1) / G, 1);
-        return (G & 7) ? G : min(G, ((n + rounds - 1) / rounds + 7) / 8 * 8);
-    };
-    // this block's place among the first g blocks, XCD by XCD; far past every tile for the others
-    auto place = [&](int g) { return (G & 7) ? bid : bid < g ? (bid & 7) * (g >> 3) + (bid >> 3) : 0x3fffffff; };
     // A chained GEMM's light tiles: one queue over the two classes, longest tiles first.  (Tile times differ by a
     // factor of two with the load on the memory, so no static plan ends evenly: a layer of 22 touched experts, one of
     // 2311 rows, ended its GMM1 between 66 and 303 us under round-robin, against 175 us of work per block.)
@@ -1595,7 +1634,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     int ge = G;
     if (n0 == 0)
         ge = ROLE == SYNC_PRODUCE && n1 + n2 + n3 >= G ? G : blocks_for(n1 + n2 + n3);
-    int nfree = ge, rank = place(ge);
+    int nfree = ge, rank = place_among(ge);
     bool is_free = rank < ge;
     if (n0 > 0 && n0 < G && (G & 7) == 0) {
         // Fewer heavy tiles than blocks.  They are split evenly over the 8 XCDs (XCD x takes the run
@@ -1605,7 +1644,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         auto heavy_in = [&](int x) { return max(0, min(hx, n0 - x * hx)); };
         const int len = heavy_in(xcd);
         if (slot < len) {
-            gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, 0x3fffffff, xcd * hx + slot, (len - slot + S - 1) / S, S, wv);
+            gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, G_NOWHERE, xcd * hx + slot, (len - slot + S - 1) / S, S, wv);
             lds_sync();  // every wave is done with the first class's ring
         }
         int free_before = 0, busy_before = 0;
@@ -1650,7 +1689,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
             free_end += f ? cost : 0;
             busy_end += f ? 0 : cost;
         }
-        const int mine = is_free ? nf : nb, r = rank < ng ? (rank - at + ng) % ng : 0x3fffffff;
+        const int mine = is_free ? nf : nb, r = rank < ng ? (rank - at + ng) % ng : G_NOWHERE;
         // (divisions leave their results in vector registers: scalar ones, as above)
         rs = __builtin_amdgcn_readfirstlane((is_free ? 0 : nf) + r);
         rn = __builtin_amdgcn_readfirstlane(max(0, (mine - r + ng - 1) / max(ng, 1)));
@@ -1661,13 +1700,13 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     int rs, rn;
     if (n1 > 0) {
         light(n1, 14, rs, rn);
-        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
+        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
         lds_sync();
     }
     if constexpr (DT == DT_INT8) {
         if (n2 > 0) {
             light(n2, 14, rs, rn);
-            gmm_body<DT, EPI, CLS_128S, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
+            gmm_body<DT, EPI, CLS_128S, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
         }
     }
     if constexpr (HAS32) {
@@ -1675,7 +1714,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
             light(n3, EPI == EPI_PLAIN ? 5 : 11, rs, rn);
             if (!KEEP && wv >= Tile<32>::NWAVES)
                 return;  // the 32-row tile's four waves go on (a barrier only counts the waves still running)
-            gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, 0x3fffffff, rs, rn, ng, wv);
+            gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
         }
     }
 }
@@ -1726,26 +1765,49 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     // first GMM2 tiles (the first experts) depend only on GMM1's first round.
     const int pos = xcd_position(), G = gridDim.x;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    int t1;
+    int t1, ge;
     {
         const GmmArgs p1 = chain_params()->g1;
-        build_group_tables<Tile<32>::THREADS>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                              ClassRanges{{0, 0, 0, 0}, {0, 0, 0, 0x7fffffff}});
-        t1 = gt->template end<CLS_32>(p1.L - 1) * (p1.N / 2 / 128);
-        gmm_body<DT, EPI1, CLS_32, SYNC_PRODUCE, true, W_BY_TILE>(p1, gt, pos, 0, 0, 1, wv);
+        const int ntn = p1.N / 2 / 128;
+        build_group_tables<Tile<32>::THREADS, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
+                                                    small_ranges(), 0, ClassRanges{}, G / ntn);
+        const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p1.L - 1)) * ntn;
+        const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p1.L - 1)) * ntn;
+        t1 = n64 + n32;
+        ge = t1 < G ? blocks_for(t1) : G;  // (few tiles spread over the XCDs)
+        const int rank = place_among(ge);
+        auto rounds = [&](int r, int n) { return __builtin_amdgcn_readfirstlane(r < ge ? (n - r + ge - 1) / ge : 0); };
+        if (n64 > 0) {
+            gmm_body<DT, EPI1, CLS_64, SYNC_PRODUCE, true, policy64(DT)>(p1, gt, G_NOWHERE, rank, rounds(rank, n64), ge, wv);
+            lds_sync();
+        }
+        const int r32 = __builtin_amdgcn_readfirstlane(rank < ge ? (rank + ge - n64 % ge) % ge : G_NOWHERE);
+        gmm_body<DT, EPI1, CLS_32, SYNC_PRODUCE, true>(p1, gt, G_NOWHERE, r32, rounds(r32, n32), ge, wv);
     }
     lds_sync();
     const GmmArgs p2 = chain_params()->g2;
-    const int r1 = t1 % G, nfree = r1 ? G - r1 : 0;
-    const bool is_free = nfree > 0 && pos >= r1;
+    // the blocks with one GMM1 tile fewer: nfree, this one number fr of them
+    const bool few = ge < G;
+    const int r1 = few ? ge : t1 % G, nfree = r1 ? G - r1 : 0;
+    const int fr = (few ? (int)blockIdx.x : pos) - r1;
+    const bool is_free = nfree > 0 && fr >= 0;
     constexpr int BN2 = small_bn(32, EPI_PLAIN);
+    const int m64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p2.L - 1)) * (p2.N / BN2);
+    const int m32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p2.L - 1)) * (p2.N / BN2);
     // (never more than spreads GMM2's tiles over the free blocks: with few tiles a run would leave most of them idle;
     // one token through 2 of 8 bf16 experts, H = 1024: 16 GMM2 tiles on 16 blocks instead of 4)
-    const int t2 = gt->template end<CLS_32>(p2.L - 1) * (p2.N / BN2);
-    const int R = max(1, min((GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K),
-                             nfree ? (t2 + nfree - 1) / nfree : 1));
-    gmm_body<DT, EPI_PLAIN, CLS_32, SYNC_CONSUME, true, W_BY_TILE>(p2, gt, R * nfree + pos, is_free ? (pos - r1) * R : 0,
-                                                          is_free ? R : 0, 1, wv);
+    const int R = __builtin_amdgcn_readfirstlane(
+        max(1, min((GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K),
+                   nfree ? (m64 + m32 + nfree - 1) / nfree : 1)));
+    // the block's tiles of both classes in turn: the run [run, run + rn), then next, next + G, ...
+    const int run = is_free ? fr * R : 0, rn = is_free ? R : 0, next = R * nfree + pos;
+    if (m64 > 0) {
+        gmm_body<DT, EPI_PLAIN, CLS_64, SYNC_CONSUME, true, policy64(DT)>(p2, gt, next, run, min(rn, max(m64 - run, 0)), 1, wv);
+        lds_sync();
+    }
+    const int skip = max(m64 - run, 0), after = max(m64 - next + G - 1, 0) / G;
+    gmm_body<DT, EPI_PLAIN, CLS_32, SYNC_CONSUME, true>(p2, gt, __builtin_amdgcn_readfirstlane(next + after * G - m64),
+                                                        max(run - m64, 0), max(rn - skip, 0), 1, wv);
 }
 
 // Per-device launch state: the CU count and whether a kernel's dynamic-LDS limit has been raised.
