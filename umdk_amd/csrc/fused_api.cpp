@@ -3,7 +3,9 @@
 // fused_deep_moe.h:355-448) on one GPU, composed from the path's kernels:
 //   prepare ids (x_active_mask, local expert range) -> layout -> count
 //   exchange -> quantised dispatch -> GMM1+SwiGLU -> GMM2 -> combine,
-//   plus the optional shared expert on all tokens.  At decode sizes
+//   plus the optional shared expert on all tokens: where it is as wide as the
+//   routed ones, one more expert of the same GEMM launches, its rows after the
+//   routed rows (a launch pair of its own leaves most of the GPU idle).  At decode sizes
 //   (batch*topk <= 2048, bf16 or fp8) the first four stages are one launch
 //   (every block computes the layout in LDS), dispatch writes the combine's
 //   row map, and GMM1 and GMM2 run as one chained launch (each GMM2 tile waits
@@ -48,6 +50,7 @@ struct Carve {
 
 struct FusedLayout {
     uint64_t ids, layout_ws, counts, send_off, recv_cnt, total, sti, ex, xs, eidx, h, hs, y, inv, hf, amax, ready;
+    uint64_t groups;
     uint64_t sh_x, sh_xs, sh_h, sh_hs, sh_gl, sh_hf, sh_amax;
     uint64_t bytes;
 };
@@ -58,11 +61,12 @@ static uint64_t scale_bytes(int dt, uint64_t cols)
     return dt == cam::DT_FP8 ? cols / 128 * 4 : dt == cam::DT_INT8 ? 4 : 0;
 }
 
-FusedLayout plan_fused(int T, int H, int K, int L, int I, int Ish, int dt, bool shared)
+// merged: the shared expert's T rows follow the routed ones (shared: it has buffers of its own)
+FusedLayout plan_fused(int T, int H, int K, int L, int I, int Ish, int dt, bool shared, bool merged)
 {
     Carve c;
     FusedLayout f{};
-    const uint64_t N = (uint64_t)T * K;
+    const uint64_t N = (uint64_t)T * K, MR = N + (merged ? T : 0), GL = L + (merged ? 1 : 0);
     const uint64_t esz = dt == cam::DT_BF16 ? 2 : 1;
     const bool int8 = dt == cam::DT_INT8;
     f.ids = c.take(4 * N);
@@ -72,16 +76,17 @@ FusedLayout plan_fused(int T, int H, int K, int L, int I, int Ish, int dt, bool 
     f.recv_cnt = c.take(4 * (uint64_t)L);
     f.total = c.take(4);
     f.sti = c.take(4 * N);
-    f.ex = c.take(N * H * esz);
-    f.xs = c.take(N * scale_bytes(dt, H));
+    f.ex = c.take(MR * H * esz);
+    f.xs = c.take(MR * scale_bytes(dt, H));
     f.eidx = c.take(12 * N);
-    f.h = c.take(N * I * esz);
-    f.hs = c.take(N * scale_bytes(dt, I));
+    f.h = c.take(MR * I * esz);
+    f.hs = c.take(MR * scale_bytes(dt, I));
     f.y = c.take(N * H * 2);
     f.inv = c.take(4 * N);
-    f.hf = c.take(int8 ? N * I * 4 : 0);  // int8: fp32 h and its row maxima before the requantisation
-    f.amax = c.take(int8 ? N * (I / cam::GMM_AMAX_COLS) * 4 : 0);  // partial row maxima of h
-    f.ready = c.take(int8 ? 0 : 4 * (uint64_t)cam::gmm_chain_counters((int)N, L));  // chained GEMMs' counters
+    f.hf = c.take(int8 ? MR * I * 4 : 0);  // int8: fp32 h and its row maxima before the requantisation
+    f.amax = c.take(int8 ? MR * (I / cam::GMM_AMAX_COLS) * 4 : 0);  // partial row maxima of h
+    f.ready = c.take(int8 ? 0 : 4 * (uint64_t)cam::gmm_chain_counters((int)MR, (int)GL));  // chained GEMMs' counters
+    f.groups = c.take(merged ? 8 * GL : 0);
     if (shared) {
         f.sh_x = c.take((uint64_t)T * H * esz);
         f.sh_xs = c.take((uint64_t)T * scale_bytes(dt, H));
@@ -195,8 +200,15 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
     const int I = (int)(gmm1HiddenSize / 2), Ish = (int)(shareGmm1HiddenSize / 2);
     const int dt = (int)weightDtype;  // CAMHIP_DTYPE_* equal cam::DT_*
     const bool int8 = dt == cam::DT_INT8;
-    const FusedLayout f = plan_fused(T, H, K, L, I, shared ? Ish : 0, dt, shared);
     const int N = T * K;
+    // A shared expert of the routed experts' width joins their GEMMs as group L, its rows (every token) after the
+    // routed ones (128 tokens, 32 of 256 int8 experts, H = 7168, I = 2048, smooth scales: the decode step 272 us
+    // against 347 us with its own dispatch, GEMMs and requantisation); one of another width, and a batch past the
+    // single-launch layouts, keeps its own launches.
+    const bool merged = shared && Ish == I && N <= 8192 && L < 512 &&
+                        (int64_t)(N + T) * std::max(H, I) * (dt == cam::DT_BF16 ? 2 : 1) < (int64_t)1 << 32;
+    const FusedLayout f = plan_fused(T, H, K, L, I, shared ? Ish : 0, dt, shared && !merged, merged);
+    const int MR = N + (merged ? T : 0), GL = L + (merged ? 1 : 0);
     const int q = dt == cam::DT_FP8 ? cam::QUANT_FP8_BLOCK : int8 ? cam::QUANT_INT8_FUSED : cam::QUANT_NONE;
     const int epi1 = dt == cam::DT_FP8 ? cam::EPI_SWIGLU_FP8 : int8 ? cam::EPI_SWIGLU_F32AMAX : cam::EPI_SWIGLU_BF16;
     // GMM1 + SwiGLU: int8 writes fp32 h and row maxima, then requantises per token
@@ -220,9 +232,11 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
         if (T == 0) {  // no tokens: no expert receives any
             return cam::launch_fill_i64(expertTokenNums, 0, L, s);
         }
-        cam::GmmArgs g1{(const uint8_t *)P(f.ex), (const float *)P(f.xs), expertTokenNums, L, N, H, 2 * I,
+        int64_t *groups = merged ? (int64_t *)P(f.groups) : nullptr;
+        const int64_t *gl = merged ? groups : expertTokenNums;
+        cam::GmmArgs g1{(const uint8_t *)P(f.ex), (const float *)P(f.xs), gl, GL, MR, H, 2 * I,
                         (const uint8_t *)gmm1Weight, gmm1WeightScale, (uint8_t *)P(f.h), (float *)P(f.hs)};
-        cam::GmmArgs g2{(const uint8_t *)P(f.h), (const float *)P(f.hs), expertTokenNums, L, N, I, H,
+        cam::GmmArgs g2{(const uint8_t *)P(f.h), (const float *)P(f.hs), gl, GL, MR, I, H,
                         (const uint8_t *)gmm2Weight, gmm2WeightScale, (uint8_t *)P(f.y), nullptr};
         if (wlist) {
             g1.Wl = (const uint8_t *const *)gmm1Weight;
@@ -230,23 +244,32 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
             g2.Wl = (const uint8_t *const *)gmm2Weight;
             g2.Wsl = (const float *const *)gmm2WeightScale;
         }
+        if (merged) {
+            g1.ex = g2.ex = L;
+            g1.Wx = (const uint8_t *)shareGmm1Weight;
+            g1.Wsx = shareGmm1WeightScale;
+            g2.Wx = (const uint8_t *)shareGmm2Weight;
+            g2.Wsx = shareGmm2WeightScale;
+            g2.Cx = (uint8_t *)shareOutput;
+        }
         // GMM1 -> GMM2 as one launch where a chained kernel exists; its readiness counters start at zero
         const bool chained = cam::gmm_chain_supported(g1, g2, dt);
         int32_t *ready = (int32_t *)P(f.ready);
-        const int nready = chained ? cam::gmm_chain_counters(N, L) : 0;
+        const int nready = chained ? cam::gmm_chain_counters(MR, GL) : 0;
         // decode sizes with bf16 or fp8 rows: id preparation, layout, count exchange and the dispatch in one
         // launch (which also clears the counters)
         const bool one_launch = !int8 && cam::dispatch_decode_fits(T, K, L);
         if (one_launch) {
-            HIP_TRY(cam::launch_dispatch_decode(expertIds, xActiveMask, x, T, H, K, L, N, q, P(f.ex), (float *)P(f.xs),
+            HIP_TRY(cam::launch_dispatch_decode(expertIds, xActiveMask, x, T, H, K, L, MR, q, P(f.ex), (float *)P(f.xs),
                                                 (int32_t *)P(f.eidx), (int32_t *)P(f.inv), true, counts, send_off,
-                                                recv_cnt, (int32_t *)P(f.total), expertTokenNums, s, ready, nready));
+                                                recv_cnt, (int32_t *)P(f.total), expertTokenNums, s, ready, nready,
+                                                groups));
         } else if (N <= 8192) {
             // decode sizes: id preparation, layout and count exchange in one launch (which also clears the
             // counters)
             HIP_TRY(cam::launch_layout_small(expertIds, xActiveMask, T, K, L, ids, counts, (int32_t *)P(f.sti),
                                              send_off, recv_cnt, (int32_t *)P(f.total), expertTokenNums, s, ready,
-                                             nready));
+                                             nready, groups));
         } else {
             if (chained)
                 HIP_TRY(cam::launch_fill_i32(ready, 0, nready, s));
@@ -258,9 +281,11 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
         // dispatch also writes the combine's row map (inv), so the combine is a single gather; fp8 block
         // scales come out k-major, the layout GMM1 reads
         if (!one_launch)
-            HIP_TRY(cam::launch_dispatch(x, ids, send_off, (int32_t *)P(f.sti), T, H, K, L, 0, N, q, P(f.ex),
+            HIP_TRY(cam::launch_dispatch(x, ids, send_off, (int32_t *)P(f.sti), T, H, K, L, 0, MR, q, P(f.ex),
                                          (float *)P(f.xs), (int32_t *)P(f.eidx), s, (int32_t *)P(f.inv),
-                                         expertSmoothScales, true));
+                                         expertSmoothScales, true, nullptr, 0, nullptr, false,
+                                         merged ? (const int32_t *)P(f.total) : nullptr,
+                                         merged ? shareSmoothScales : nullptr));
         if (chained) {
             HIP_TRY(cam::launch_gmm_chain(g1, g2, dt, ready, s));
         } else {
@@ -270,7 +295,7 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
         HIP_TRY(cam::launch_combine_gather((const uint16_t *)P(f.y), (const int32_t *)P(f.eidx), N,
                                            recv_cnt + (L - 1), expertScales, T, K, H, output,
                                            (const int32_t *)P(f.inv), s));
-        if (shared) {
+        if (shared && !merged) {
             // shared expert on every token: x quantised in token order, one group of T rows
             int64_t *gl = (int64_t *)P(f.sh_gl);
             HIP_TRY(cam::launch_fill_i64(gl, T, 1, s));

@@ -29,6 +29,12 @@ struct GmmArgs {
     // ([N/128, K/128] fp8, [N] int8); when set, W and Ws are not read.
     const uint8_t *const *Wl = nullptr;
     const float *const *Wsl = nullptr;
+    // A last expert of its own (optional; group ex = L - 1): weights Wx and scales Wsx in place of W's and Wl's next
+    // entry, and for the plain GEMM the output Cx, which holds that expert's rows alone.
+    int ex = -1;
+    const uint8_t *Wx = nullptr;
+    const float *Wsx = nullptr;
+    uint8_t *Cx = nullptr;
 };
 
 hipError_t launch_gmm(const GmmArgs &a, int dt, int epi, hipStream_t s);

@@ -214,7 +214,8 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // the counts.  Only experts with a row count in a class's [lo, hi) get tiles of that class (a launch may
 // split the experts between tile heights); the row offsets count every expert (they locate segments in
 // dispatch order).
-template <int GTHREADS, bool FOUR_WAVES = false>
+// MASK: the classes the kernel has (the others cost the scan nothing).
+template <int GTHREADS, int MASK, bool FOUR_WAVES = false>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
                                    ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{},
                                    int few_tiles = 0)
@@ -222,39 +223,42 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
     constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(FOUR_WAVES ? CLS_64 : CLS_128M),
                                    FOUR_WAVES ? 32 : class_bm(2), class_bm(3)};
-    const int tid = threadIdx.x;
-    const int per = (L + GTHREADS - 1) / GTHREADS;
-    constexpr int NWV = GTHREADS / 64;
-    const int lane = tid & 63, wv = tid >> 6;
+    constexpr int PER = (G_MAX_L + GTHREADS - 1) / GTHREADS, NWV = GTHREADS / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    auto used = [](int k) { return k == G_NCLASS || ((MASK >> k) & 1); };
+    int rows[PER];  // experts PER tid + q, read once
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        rows[q] = tid * PER + q < L ? (int)group_list[tid * PER + q] : 0;
     int cnt[NQ] = {};
     auto add = [&](int c, int *v) {
 #pragma unroll
         for (int k = 0; k < G_NCLASS; ++k)
-            v[k] += (c >= cr.lo[k] && c < cr.hi[k]) ? (c + BMS[k] - 1) / BMS[k] : 0;
+            if (used(k))
+                v[k] += (c >= cr.lo[k] && c < cr.hi[k]) ? (c + BMS[k] - 1) / BMS[k] : 0;
         v[G_NCLASS] += c;
     };
     if (heavy_rows > 0) {  // cr_heavy where some expert holds that many rows
-        int any = 0;
-        for (int q = 0; q < per; ++q)
-            any |= tid * per + q < L && group_list[tid * per + q] >= heavy_rows;
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            any |= rows[q] >= heavy_rows;
         int *flag = scratch + NQ * NWV;
         if (lane == 0)
             flag[wv] = 0;
         if (any)
             flag[wv] = 1;
         __syncthreads();
-        any = 0;
+        int f = 0;
 #pragma unroll
         for (int v = 0; v < NWV; ++v)
-            any |= flag[v];
-        if (any)
+            f |= flag[v];
+        if (f)
             cr = cr_heavy;
     }
-    for (int q = 0; q < per; ++q) {
-        const int e = tid * per + q;
-        if (e < L)
-            add((int)group_list[e], cnt);
-    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        add(rows[q], cnt);
     // exclusive scan: within each wave by lane shuffles, then over the waves' totals
     int inc[NQ];
 #pragma unroll
@@ -264,6 +268,8 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
     for (int d = 1; d < 64; d <<= 1) {
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
+            if (!used(k))
+                continue;
             const int u = __shfl_up(inc[k], d, 64);
             if (lane >= d)
                 inc[k] += u;
@@ -281,7 +287,7 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
         int ex = inc[k] - cnt[k];
 #pragma unroll
         for (int v = 0; v < NWV; ++v)
-            ex += v < wv ? scratch[k * NWV + v] : 0;
+            ex += used(k) && v < wv ? scratch[k * NWV + v] : 0;
         run[k] = ex;
     }
     bool few = false;
@@ -292,10 +298,11 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
             all32 += scratch[2 * NWV + v];
         few = all32 <= few_tiles;
     }
-    for (int q = 0; q < per; ++q) {
-        const int e = tid * per + q;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = tid * PER + q;
+        add(rows[q], run);
         if (e < L) {
-            add((int)group_list[e], run);
             if constexpr (FOUR_WAVES) {
                 gt.tile_end[CLS_256][e] = 0;
                 gt.tile_end[CLS_128M][e] = few ? 0 : run[CLS_128M];
@@ -544,7 +551,10 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         c.active = !spect && c.row0 + wm * WM < c.seg1;
         c.nt = mt_e == 1;
 
-        if (p.Wl) {  // separated weights: one allocation per expert, pointers read by scalar loads (a vector
+        if (e == p.ex) {
+            c.wbase = p.Wx;
+            c.wsb = p.Wsx;
+        } else if (p.Wl) {  // separated weights: one allocation per expert, pointers read by scalar loads (a vector
                      // load here would make the tile switch wait for every DMA in flight)
             c.wbase = reinterpret_cast<const uint8_t *>(
                 ((const __attribute__((address_space(4))) uint64_t *)p.Wl)[e]);
@@ -657,12 +667,15 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         const int row0 = c.row0, seg1 = c.seg1, n0 = c.n0;
         const int lid = lane_here<FRESH>(), l16 = lid & 15, lg = lid >> 4;
         if constexpr (EPI == EPI_PLAIN) {
+            uint16_t *out = reinterpret_cast<uint16_t *>(p.C);
+            if (c.e == p.ex)
+                out = reinterpret_cast<uint16_t *>(p.Cx) - (size_t)__builtin_amdgcn_readfirstlane(row_off(c.e)) * p.N;
 #pragma unroll
             for (int i = 0; i < IF; ++i) {
                 const int m = row0 + wm * WM + i * 16 + l16;
                 if (m >= seg1)
                     continue;
-                uint16_t *crow = reinterpret_cast<uint16_t *>(p.C) + (size_t)m * p.N + n0 + wn * WN + 4 * lg;
+                uint16_t *crow = out + (size_t)m * p.N + n0 + wn * WN + 4 * lg;
 #pragma unroll
                 for (int j = 0; j < JF; ++j) {
                     u32x2 v;
@@ -1520,7 +1533,7 @@ template <int DT, int EPI> __global__ __launch_bounds__(256, DT == DT_INT8 ? 1 :
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / small_bn(32, EPI);
-    build_group_tables<Tile<32>::THREADS, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(), 0,
+    build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(), 0,
                                                 ClassRanges{}, (int)gridDim.x / ntn);
     const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p.L - 1)) * ntn;
     const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn;
@@ -1726,8 +1739,9 @@ template <int DT, int EPI> __global__ __launch_bounds__(512, 1) void gmm_kernel_
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const bool tall = big_tall(p.allow256, p.K, DT);
     // every class's expert table, from one read of the counts
-    build_group_tables<GMAX_THREADS>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
-                                     big_ranges<DT>(tall, false), tall ? G_HEAVY_ROWS : 0, big_ranges<DT>(tall, true));
+    build_group_tables<GMAX_THREADS, DT == DT_INT8 ? 7 : 11>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
+                                     big_ranges<DT>(tall, false),
+                                     DT == DT_INT8 && tall ? G_HEAVY_ROWS : 0, big_ranges<DT>(tall, true));
     big_schedule<DT, EPI, SYNC_NONE>(p, gt, wv);
 }
 
@@ -1746,7 +1760,7 @@ template <int DT, int EPI1> __global__ __launch_bounds__(512, 1) void gmm_chain_
     {
         const GmmArgs p1 = chain_params()->g1;
         tall = big_tall(p1.allow256, p1.K, DT);  // the host checked that GMM2 makes the same choice
-        build_group_tables<GMAX_THREADS>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
+        build_group_tables<GMAX_THREADS, 11>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
                                          big_ranges<DT>(tall, false));
         big_schedule<DT, EPI1, SYNC_PRODUCE>(p1, gt, wv);
     }
@@ -1769,7 +1783,7 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     {
         const GmmArgs p1 = chain_params()->g1;
         const int ntn = p1.N / 2 / 128;
-        build_group_tables<Tile<32>::THREADS, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
+        build_group_tables<Tile<32>::THREADS, 14, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
                                                     small_ranges(), 0, ClassRanges{}, G / ntn);
         const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p1.L - 1)) * ntn;
         const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p1.L - 1)) * ntn;

@@ -42,11 +42,12 @@ hipError_t launch_layout_i32(const int32_t *topk_idx, int T, int K, int E, int32
                              int32_t *send_token_idx, void *ws, hipStream_t s);
 
 // decode-sized layout + count exchange in one launch (T*K <= 8192; ids masked by `active`); it also zeroes
-// zero[0, nzero) (a later launch's counters)
+// zero[0, nzero) (a later launch's counters) and, for a shared expert that the GEMMs run as group E, writes their group
+// list groups[0, E] (tokens_per_expert, then T)
 hipError_t launch_layout_small(const int32_t *ids, const uint8_t *active, int T, int K, int E, int32_t *ids_eff,
                                int32_t *counts, int32_t *sti, int32_t *send_offset, int32_t *recv_count,
                                int32_t *total, int64_t *tokens_per_expert, hipStream_t s, int32_t *zero = nullptr,
-                               int nzero = 0);
+                               int nzero = 0, int64_t *groups = nullptr);
 
 // ---- small utilities (notify.hip)
 hipError_t launch_fill_i32(int32_t *p, int32_t v, long n, hipStream_t s);
@@ -62,7 +63,8 @@ hipError_t launch_dispatch(const uint16_t *x, const int32_t *topk_idx, const int
                            void *expand_x, float *scales, int32_t *expand_idx, hipStream_t s,
                            int32_t *inv_out = nullptr, const float *smooth = nullptr, bool kmajor_scales = false,
                            const int32_t *chunk_base = nullptr, int tpc = 0, const int32_t *chunk_rank = nullptr,
-                           bool skip_unrouted = false);
+                           bool skip_unrouted = false, const int32_t *share = nullptr,
+                           const float *share_smooth = nullptr);
 // decode sizes (dispatch_decode_fits: T*K <= 2048, E <= 512; bf16 or fp8 rows): layout + count exchange +
 // dispatch as one launch (the arguments of launch_layout_small and launch_dispatch; the ranks and effective ids
 // stay in LDS)
@@ -70,7 +72,9 @@ hipError_t launch_dispatch_decode(const int32_t *ids, const uint8_t *active, con
                                   int E, int cap, int quant_mode, void *expand_x, float *scales, int32_t *expand_idx,
                                   int32_t *inv_out, bool kmajor_scales, int32_t *counts, int32_t *send_offset,
                                   int32_t *recv_count, int32_t *total, int64_t *tokens_per_expert, hipStream_t s,
-                                  int32_t *zero, int nzero);
+                                  int32_t *zero, int nzero, int64_t *groups = nullptr);
+// (groups: as for launch_layout_small; every token then also goes to row total + t.  share: the same from a layout's
+// total; share_smooth: the int8 smooth scales of those rows)
 bool dispatch_decode_fits(int T, int K, int E);
 // (send_token_idx == nullptr: the rank within the expert is chunk_base[e * nc + t / tpc] plus chunk_rank[t * K + k],
 // the rank inside the token's chunk of tpc tokens; skip_unrouted: tokens with no pick in [0, E) read nothing, for a

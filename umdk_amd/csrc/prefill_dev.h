@@ -242,6 +242,7 @@ template <int NT> struct LayoutLds {
     int32_t count[LAYOUT_LDS_MAX_E], off[LAYOUT_LDS_MAX_E];
     int32_t wave_hist[NT / 64][LAYOUT_LDS_MAX_E];
     int32_t wave_sum[NT / 64];
+    int32_t total;
 };
 template <int NT>
 __device__ __forceinline__ void layout_lds(const int32_t *__restrict__ ids, const uint8_t *__restrict__ active, int T,
@@ -338,22 +339,29 @@ __device__ __forceinline__ void layout_lds(const int32_t *__restrict__ ids, cons
         if (e < E)
             s.off[e] = run;
         run += cnt[u];
+        if (e == E - 1)
+            s.total = run;
     }
     __syncthreads();
 }
 // The layout's global outputs (by one block): counts, send offsets, inclusive counts, the total and the int64
-// tokens per expert.
+// tokens per expert; with a shared expert also the GEMMs' group list: the same and the T rows of that expert.
 template <int NT>
 __device__ __forceinline__ void layout_lds_store(const LayoutLds<NT> &s, int E, int32_t *__restrict__ counts,
                                                  int32_t *__restrict__ send_offset, int32_t *__restrict__ recv_count,
-                                                 int32_t *__restrict__ total, int64_t *__restrict__ tokens_per_expert)
+                                                 int32_t *__restrict__ total, int64_t *__restrict__ tokens_per_expert,
+                                                 int64_t *__restrict__ groups, int T)
 {
+    if (groups && threadIdx.x == 0)
+        groups[E] = T;
     for (int e = threadIdx.x; e < E; e += NT) {
         const int32_t c = s.count[e], o = s.off[e];
         counts[e] = c;
         send_offset[e] = o;
         recv_count[e] = o + c;
         tokens_per_expert[e] = c;
+        if (groups)
+            groups[e] = c;
         if (e == E - 1)
             *total = o + c;
     }
@@ -369,9 +377,11 @@ struct RankSrc {
     const int32_t *chunk_base;
     const int32_t *chunk_rank;
     int tpc;
+    // a shared expert, which takes every token: its row of token t is *share + t, after the routed rows (else null)
+    const int32_t *share;
 };
 
-// Resolves the K destination rows of token t: lane k < K holds row(t,k) or -1.
+// Resolves the K destination rows of token t: lane k < K holds row(t,k) or -1, lane K the shared expert's row.
 __device__ __forceinline__ int dispatch_dest(const int32_t *__restrict__ topk_idx,
                                              const int32_t *__restrict__ send_offset, const RankSrc &rs, int t,
                                              int T, int K, int E, int cap, int lane)
@@ -392,6 +402,8 @@ __device__ __forceinline__ int dispatch_dest(const int32_t *__restrict__ topk_id
             dst = send_offset[e] + rs.chunk_base[(size_t)e * nc + t / rs.tpc] + rs.chunk_rank[(size_t)t * K + lane];
         }
     }
+    if (rs.share && lane == K)
+        dst = *rs.share + t;
     if (dst >= cap)  // inconsistent counts: never write outside the output
         dst = -1;
     return dst < 0 ? -1 : dst;
@@ -414,6 +426,7 @@ __device__ __forceinline__ void dispatch_wave(const uint16_t *__restrict__ x, co
 {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
+    const int ndst = K + (rs.share != nullptr);
     bool waited = false;
     // skip_unrouted (a rank holding some of the experts): a token none of whose picks is an expert of this rank
     // reads nothing, only its row-map entries are written (config 4, 32 of 256 experts local: 40% of the
@@ -445,7 +458,7 @@ __device__ __forceinline__ void dispatch_wave(const uint16_t *__restrict__ x, co
         const int dst = dispatch_dest(topk_idx, send_offset, rs, t, T, K, E, cap, lane);
         if (inv_out && j == 0 && lane < K)  // the combine's row map, so it needs no scatter pass
             inv_out[(size_t)t * K + lane] = dst;
-        for (int k = 0; k < K; ++k) {
+        for (int k = 0; k < ndst; ++k) {
             const int row = __shfl(dst, k, 64);
             if (row < 0)
                 continue;
@@ -455,7 +468,7 @@ __device__ __forceinline__ void dispatch_wave(const uint16_t *__restrict__ x, co
                 if (act1)
                     *reinterpret_cast<u32x4 *>(out + 512) = raw1;
             }
-            if (j == 0 && lane == 0 && expand_idx) {
+            if (j == 0 && lane == 0 && expand_idx && k < K) {
                 expand_idx[(size_t)row * 3 + 0] = rank;
                 expand_idx[(size_t)row * 3 + 1] = t;
                 expand_idx[(size_t)row * 3 + 2] = k;
@@ -493,7 +506,7 @@ __device__ __forceinline__ void dispatch_wave(const uint16_t *__restrict__ x, co
         for (int w = 0; w < 4; ++w)
             q[w] = f32x4_to_e4m3(f[4 * w] * inv, f[4 * w + 1] * inv, f[4 * w + 2] * inv, f[4 * w + 3] * inv);
         const int nb = H >> 7;
-        for (int k = 0; k < K; ++k) {
+        for (int k = 0; k < ndst; ++k) {
             const int row = __shfl(dst, k, 64);
             if (row < 0)
                 continue;
@@ -502,7 +515,7 @@ __device__ __forceinline__ void dispatch_wave(const uint16_t *__restrict__ x, co
                 if ((lane & 7) == 0)
                     scales[kmajor ? (size_t)(col >> 7) * cap + row : (size_t)row * nb + (col >> 7)] = bscale;
             }
-            if (j == 0 && lane == 0 && expand_idx) {
+            if (j == 0 && lane == 0 && expand_idx && k < K) {
                 expand_idx[(size_t)row * 3 + 0] = rank;
                 expand_idx[(size_t)row * 3 + 1] = t;
                 expand_idx[(size_t)row * 3 + 2] = k;
