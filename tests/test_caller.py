@@ -1,0 +1,45 @@
+"""The native caller of the C ABI (umdk_amd/_camcall.so) on the CPU: argument conversion, the library's errors, and the
+workspace it asks for.  Nothing launches: every call fails in its validation or in its allocation."""
+import pytest
+
+from umdk_amd import _lib
+
+
+def raw(name, *args, alloc=None, ws=None, have=0):
+    return getattr(_lib._calls(), name)(alloc, ws, have, 0, *args)
+
+
+def test_library_errors_keep_their_type_and_text():
+    with pytest.raises(_lib.CamHipError, match=r"^camhipMoeRouteGetWorkspaceSize failed \(\d+\): moe_route: numExperts 0"):
+        raw("camhipMoeRoute", 16, None, 4, 0, 1, 16, 16, None)
+    with pytest.raises(_lib.CamHipError, match="logits must not be NULL"):
+        raw("camhipMoeRoute", None, None, 4, 8, 2, 16, 16, None)
+    # the launch phase: a workspace too small (checked before anything runs)
+    with pytest.raises(_lib.CamHipError, match=r"^camhipDispatchLayout failed \(\d+\): dispatch_layout: workspace of 8 bytes"):
+        raw("camhipDispatchLayout", 16, 64, 1, 8, 2, None, 16, None, 16, ws=16, have=8)
+
+
+@pytest.mark.parametrize("args", [(16, None, 4.0, 8, 2, 16, 16, None), (16, None, None, 8, 2, 16, 16, None),
+                                  ("x", None, 4, 8, 2, 16, 16, None), (16, None, 4, 8, 2, 16, 16)])
+def test_wrong_arguments_are_type_errors(args):
+    with pytest.raises(TypeError):
+        raw("camhipMoeRoute", *args)
+
+
+def test_every_entry_point_is_there():
+    for name in _lib.SIGNATURES:
+        with pytest.raises(TypeError, match=name):
+            raw(name)
+
+
+def test_workspace_size_and_failed_allocation():
+    want = _lib.workspace_size("camhipDispatchLayout", 1, 64, 1, 8, 2, None, 1, None, 1)
+    seen = []
+
+    def alloc(n):
+        seen.append(n)
+        raise MemoryError("no room")
+
+    with pytest.raises(MemoryError, match="no room"):
+        raw("camhipDispatchLayout", 16, 64, 1, 8, 2, None, 16, None, 16, alloc=alloc)
+    assert seen == [want]

@@ -1,4 +1,5 @@
-"""Loader for libcamhip.so and a thin two-phase caller over its C ABI.
+"""Loader for libcamhip.so and a thin two-phase caller over its C ABI (the calls
+themselves in the extension module _camcall, built beside the library).
 
 The library must already be built (``python -m umdk_amd.build`` or
 ``__graft_entry__.build()``); there is no fallback path: a missing library or
@@ -33,6 +34,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_caller = None
 
 
 class CamHipError(RuntimeError):
@@ -70,6 +72,26 @@ def lib():
     return _lib
 
 
+def _calls():
+    global _caller
+    if _caller is None:
+        lib()  # (its missing-library message first)
+        try:
+            from . import _camcall
+        except ImportError as e:
+            raise ImportError(f"umdk_amd/_camcall.so is not built ({e}); run `python -m umdk_amd.build`") from e
+        _camcall.set_error(CamHipError)
+        _caller = _camcall
+    return _caller
+
+
+def _stream(device):
+    """The current stream's handle on `device` (None: the current device)."""
+    if isinstance(device, torch.device) and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
 def exported_symbols():
     return [n + s for n in SIGNATURES for s in ("GetWorkspaceSize", "")] + [
         "camhipGetLastErrorMsg", "camhipGetVersion"]
@@ -90,38 +112,15 @@ def ptr(t, transposed_ok=False):
 def call(name, *args, device=None, stream=None):
     """Runs one two-phase entry point: size the workspace, allocate it from
     torch's caching allocator on `device`, launch on the current stream."""
-    L = lib()
-    ws = ctypes.c_uint64(0)
-    ex = ctypes.c_void_p(0)
-    st = getattr(L, name + "GetWorkspaceSize")(*args, ctypes.byref(ws), ctypes.byref(ex))
-    if st != 0:
-        raise CamHipError(f"{name}GetWorkspaceSize failed ({st}): {L.camhipGetLastErrorMsg().decode()}")
-    buf = None
-    if ws.value > 0:
-        buf = torch.empty(ws.value, dtype=torch.uint8, device=device)
-    if stream is None:
-        stream = torch.cuda.current_stream(device).cuda_stream
-    st = getattr(L, name)(buf.data_ptr() if buf is not None else None, ws.value, ex, stream)
-    if st != 0:
-        raise CamHipError(f"{name} failed ({st}): {L.camhipGetLastErrorMsg().decode()}")
-    return buf
+    return getattr(_caller or _calls(), name)(lambda n: torch.empty(n, dtype=torch.uint8, device=device), None, 0,
+                                              _stream(device) if stream is None else stream, *args)
 
 
 def launch(name, *args, workspace=None, stream=None, device=None):
     """Like call(), but with a caller-owned workspace tensor (no allocation:
     safe inside a captured graph once the workspace is large enough)."""
-    L = lib()
-    ws = ctypes.c_uint64(0)
-    ex = ctypes.c_void_p(0)
-    st = getattr(L, name + "GetWorkspaceSize")(*args, ctypes.byref(ws), ctypes.byref(ex))
-    if st != 0:
-        raise CamHipError(f"{name}GetWorkspaceSize failed ({st}): {L.camhipGetLastErrorMsg().decode()}")
-    have = workspace.numel() * workspace.element_size() if workspace is not None else 0
-    if stream is None:
-        stream = torch.cuda.current_stream(device).cuda_stream
-    st = getattr(L, name)(workspace.data_ptr() if workspace is not None else None, have, ex, stream)
-    if st != 0:
-        raise CamHipError(f"{name} failed ({st}): {L.camhipGetLastErrorMsg().decode()}")
+    p, have = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
+    getattr(_caller or _calls(), name)(None, p, have, _stream(device) if stream is None else stream, *args)
 
 
 def sync_status(clear=False):

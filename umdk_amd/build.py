@@ -1,13 +1,15 @@
 """Builds libcamhip.so (the C-ABI library of HIP kernels for gfx950) in-tree.
 
-    python -m umdk_amd.build              # -> umdk_amd/lib/libcamhip.so
+    python -m umdk_amd.build              # -> umdk_amd/lib/libcamhip.so, umdk_amd/_camcall.so
 
 Every source is compiled by hipcc for gfx950 only; symbols are hidden except
-the extern "C" entry points declared in include/camhip.h.
+the extern "C" entry points declared in include/camhip.h.  _camcall.so is the
+Python caller of those entry points (host code, g++), linked against the library.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,6 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libcamhip.so")
+CALLER = os.path.join(HERE, "_camcall.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 COMMON = [
@@ -44,6 +47,18 @@ def _compile(src, defines=(), build_dir=BUILD):
     return obj
 
 
+def _build_caller():
+    tmp = CALLER + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(HERE, "pyext", "camcall.cpp"), "-o", tmp, "-L" + LIBDIR, "-l:libcamhip.so",
+           "-Wl,-rpath,$ORIGIN/lib", "-Wl,--allow-shlib-undefined"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building _camcall.so failed:\n" + r.stdout + r.stderr)
+    os.replace(tmp, CALLER)
+
+
 def build(verbose=True, defines=(), lib=LIB):
     """Compile every source and link `lib`.  `defines` (e.g. ["-DCAM_GMM_TIMELINE"]) build a variant,
     with its objects in a build folder of its own."""
@@ -59,6 +74,8 @@ def build(verbose=True, defines=(), lib=LIB):
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
     os.replace(tmp, lib)
+    if lib == LIB:
+        _build_caller()
     if verbose:
         print(f"built {lib}")
     return lib

@@ -90,16 +90,14 @@ def get_dispatch_layout(topk_idx, num_experts, num_ranks):
 def _notify(num_tokens_per_expert, T, device):
     E = num_tokens_per_expert.shape[0]
     i32 = dict(dtype=torch.int32, device=device)
-    send_offset = torch.empty(E, **i32)
+    offsets = torch.empty(2 * E + 1, **i32)  # send offsets, recv offsets, max_bs: read by the dispatch only
     total = torch.empty(1, **i32)
     recv_count = torch.empty(E, **i32)
-    recv_offset = torch.empty(E, **i32)
-    max_bs = torch.empty(1, **i32)
     rtpe = torch.empty(E, dtype=torch.int64, device=device)
-    _lib.call("camhipNotifyDispatch", _lib.ptr(num_tokens_per_expert), E, T, 1, 0, _lib.ptr(send_offset),
-              _lib.ptr(total), _lib.ptr(recv_count), _lib.ptr(recv_offset), _lib.ptr(max_bs), _lib.ptr(rtpe),
-              device=device)
-    return send_offset, total, recv_count, recv_offset, rtpe
+    send = _lib.ptr(offsets)
+    _lib.call("camhipNotifyDispatch", _lib.ptr(num_tokens_per_expert), E, T, 1, 0, send, _lib.ptr(total),
+              _lib.ptr(recv_count), send + 4 * E, send + 8 * E, _lib.ptr(rtpe), device=device)
+    return offsets, total, recv_count, rtpe
 
 
 def moe_dispatch_prefill(x, topk_idx, topk_weights, num_tokens_per_expert, send_token_idx_small, group_ep, rank,
@@ -136,7 +134,7 @@ def moe_dispatch_prefill(x, topk_idx, topk_weights, num_tokens_per_expert, send_
     _check(ti.shape[0] == T and send_token_idx_small.shape[0] == T, "moe_dispatch_prefill: token count mismatch")
     _check(topk_weights.shape[1] == K and send_token_idx_small.shape[1] == K, "moe_dispatch_prefill: topk mismatch")
     dev = x.device
-    send_offset, total, recv_count, recv_offset, rtpe = _notify(num_tokens_per_expert, T, dev)
+    offsets, total, recv_count, rtpe = _notify(num_tokens_per_expert, T, dev)
     n_recv = int(total.item())
     n_rows = max(n_recv, 1)
     if quant_mode == QUANT_NONE:
@@ -150,9 +148,10 @@ def moe_dispatch_prefill(x, topk_idx, topk_weights, num_tokens_per_expert, send_
         scales = torch.empty((n_rows, H // 128), dtype=torch.float32, device=dev)
     expand_idx = torch.empty(n_rows * 3, dtype=torch.int32, device=dev)
     sti = send_token_idx_small if send_token_idx_small.dtype == torch.int32 else send_token_idx_small.to(torch.int32)
-    _lib.call("camhipMoeDispatchNormal", _lib.ptr(x), _lib.ptr(ti), _lib.ptr(send_offset), _lib.ptr(sti.contiguous()),
-              _lib.ptr(recv_offset), _lib.ptr(recv_count), T, H, K, 1, 0, E, quant_mode, n_rows, _lib.ptr(expand_x),
-              _lib.ptr(scales), _lib.ptr(expand_idx), None, device=dev)
+    send = _lib.ptr(offsets)
+    _lib.call("camhipMoeDispatchNormal", _lib.ptr(x), _lib.ptr(ti), send, _lib.ptr(sti.contiguous()), send + 4 * E,
+              _lib.ptr(recv_count), T, H, K, 1, 0, E, quant_mode, n_rows, _lib.ptr(expand_x), _lib.ptr(scales),
+              _lib.ptr(expand_idx), None, device=dev)
     return expand_x, scales, expand_idx, recv_count, rtpe
 
 

@@ -1,0 +1,148 @@
+// Python caller of the two-phase C ABI (include/camhip.h): one extension function per entry point that converts its
+// arguments, sizes the workspace, has it allocated and launches.  Through ctypes the two calls of an operator with some
+// thirty arguments cost 8 us of host time, as much as its launches, and the smallest operator calls are bound by the
+// host (one token through moe_route and fused_deep_moe: 39 us a pass through ctypes, 34 us through this; the five-operator
+// chain at T = 1021: 90 and 75 us).
+//
+// name(alloc, workspace, workspace_bytes, stream, *args) -> buffer or None
+//   args: the GetWorkspaceSize arguments (pointers as int or None, sizes as int), without the two outputs;
+//   alloc: called with the workspace size when it is not 0, returns a tensor (its data_ptr is used and the tensor is
+//          returned); None: the caller's workspace is used;
+//   a failed call raises the exception set by set_error with the library's message.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <tuple>
+#include <type_traits>
+#include <utility>
+
+#include "camhip.h"
+
+namespace {
+
+PyObject *g_error = nullptr;
+
+template <typename A> bool convert(PyObject *o, A &out)
+{
+    if constexpr (std::is_pointer_v<A>) {
+        if (o == Py_None) {
+            out = nullptr;
+            return true;
+        }
+        if (!PyLong_Check(o)) {
+            PyErr_SetString(PyExc_TypeError, "a pointer argument must be an int or None");
+            return false;
+        }
+        out = (A)PyLong_AsVoidPtr(o);
+    } else {
+        if (!PyLong_Check(o)) {
+            PyErr_SetString(PyExc_TypeError, "a size argument must be an int");
+            return false;
+        }
+        out = (A)PyLong_AsLongLong(o);
+    }
+    return !PyErr_Occurred();
+}
+
+PyObject *failed(const char *name, const char *phase, int status)
+{
+    PyErr_Format(g_error ? g_error : PyExc_RuntimeError, "%s%s failed (%d): %s", name, phase, status,
+                 camhipGetLastErrorMsg());
+    return nullptr;
+}
+
+using RunFn = camhipStatus (*)(void *, uint64_t, camhipExecutor *, void *);
+constexpr Py_ssize_t FIXED = 4;
+
+template <typename... P, size_t... I>
+PyObject *invoke(const char *name, camhipStatus (*get)(P...), RunFn run, PyObject *const *argv, Py_ssize_t n,
+                 std::index_sequence<I...>)
+{
+    if (n != FIXED + (Py_ssize_t)sizeof...(I)) {
+        PyErr_Format(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, (Py_ssize_t)sizeof...(I), n - FIXED);
+        return nullptr;
+    }
+    std::tuple<P...> a{};
+    void *ws = nullptr, *stream = nullptr;
+    int64_t have = 0;
+    if (!convert(argv[1], ws) || !convert(argv[2], have) || !convert(argv[3], stream) ||
+        !(convert(argv[FIXED + I], std::get<I>(a)) && ...))
+        return nullptr;
+    uint64_t need = 0;
+    camhipExecutor *ex = nullptr;
+    std::get<sizeof...(I)>(a) = &need;
+    std::get<sizeof...(I) + 1>(a) = &ex;
+    int st = std::apply(get, a);
+    if (st != CAMHIP_SUCCESS)
+        return failed(name, "GetWorkspaceSize", st);
+    PyObject *buf = nullptr;
+    if (argv[0] != Py_None && need > 0) {
+        PyObject *size = PyLong_FromUnsignedLongLong(need);
+        buf = size ? PyObject_CallOneArg(argv[0], size) : nullptr;
+        Py_XDECREF(size);
+        PyObject *p = buf ? PyObject_CallMethod(buf, "data_ptr", nullptr) : nullptr;
+        const bool ok = p && convert(p, ws);
+        Py_XDECREF(p);
+        if (!ok) {
+            Py_XDECREF(buf);
+            camhipReleaseExecutor(ex);
+            return nullptr;
+        }
+        have = (int64_t)need;
+    }
+    Py_BEGIN_ALLOW_THREADS
+    st = run(ws, (uint64_t)have, ex, stream);
+    Py_END_ALLOW_THREADS
+    if (st != CAMHIP_SUCCESS) {
+        Py_XDECREF(buf);
+        return failed(name, "", st);
+    }
+    if (buf)
+        return buf;
+    Py_RETURN_NONE;
+}
+
+template <typename... P>
+PyObject *entry(const char *name, camhipStatus (*get)(P...), RunFn run, PyObject *const *argv, Py_ssize_t n)
+{
+    return invoke(name, get, run, argv, n, std::make_index_sequence<sizeof...(P) - 2>{});
+}
+
+#define ENTRIES(X)                                                                                                   \
+    X(camhipMoeRoute)                                                                                                \
+    X(camhipDispatchLayout)                                                                                          \
+    X(camhipNotifyDispatch)                                                                                          \
+    X(camhipMoeDispatchNormal)                                                                                       \
+    X(camhipMoeCombineNormal)                                                                                        \
+    X(camhipGroupedMatmulSwiglu)                                                                                     \
+    X(camhipGroupedMatmul)                                                                                           \
+    X(camhipFusedDeepMoe)                                                                                            \
+    X(camhipMoePrefillDispatch)                                                                                      \
+    X(camhipMoePrefillCombine)                                                                                       \
+    X(camhipMoeExperts)
+
+#define DEFINE(f)                                                                                                    \
+    PyObject *py_##f(PyObject *, PyObject *const *argv, Py_ssize_t n)                                                \
+    {                                                                                                                \
+        if (n < FIXED) {                                                                                             \
+            PyErr_SetString(PyExc_TypeError, #f ": alloc, workspace, workspace_bytes and stream come first");        \
+            return nullptr;                                                                                          \
+        }                                                                                                            \
+        return entry(#f, f##GetWorkspaceSize, f, argv, n);                                                           \
+    }
+ENTRIES(DEFINE)
+
+PyObject *set_error(PyObject *, PyObject *type)
+{
+    Py_INCREF(type);
+    Py_XSETREF(g_error, type);
+    Py_RETURN_NONE;
+}
+
+#define METHOD(f) {#f, (PyCFunction)(void (*)(void))py_##f, METH_FASTCALL, nullptr},
+PyMethodDef g_methods[] = {ENTRIES(METHOD){"set_error", set_error, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_camcall", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__camcall(void) { return PyModule_Create(&g_module); }
