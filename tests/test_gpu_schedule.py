@@ -16,6 +16,9 @@ PREFILL = [
     ([384, 700] * 9 + EDGES, 2048, 2048),               # more heavy tiles than blocks
     ([40, 20, 130] * 12, 2048, 2048),                   # several rounds of light tiles through the queue
     (EDGES, 256, 384),                                  # reductions of 2 and 3 k-steps: no tile primes the next
+    # heavy experts alone: the last round of the two calls' 256-row tiles as halves (the chained launch keeps them whole)
+    ([384, 700, 641], 2048, 2048),                      # the only round
+    ([2304, 2290], 2048, 2048),                         # after a full one
 ]
 
 
@@ -48,7 +51,7 @@ def test_chained_decode_tiles(lib, dt, counts):  # noqa: F811
     assert lib.sync_status() == 0
 
 
-@pytest.mark.parametrize("counts", [EDGES, EDGES + [384, 900], [2100, 40, 2100, 150, 3, 129, 128]])
+@pytest.mark.parametrize("counts", [EDGES, EDGES + [384, 900], [2100, 40, 2100, 150, 3, 129, 128], [384, 0, 900]])
 def test_int8_tiles_at_class_edges(counts):
     # int8 x int8 sums in fp64 are exact (|sum| < 2^53), then the kernel's own fp32 sequence and bf16 rounding
     import umdk_amd  # noqa: F401

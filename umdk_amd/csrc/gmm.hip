@@ -450,7 +450,8 @@ constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? 
 
 template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS)>
 __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gtab, int first, int rs = 0, int rn = 0,
-                                        int rstride = 1, int wv = -1, const TileQueue &tq = TileQueue{})
+                                        int rstride = 1, int wv = -1, const TileQueue &tq = TileQueue{},
+                                        int half0 = -1)
 {
     constexpr int BM = class_bm(CLS);
     using TC = Tile<BM, small_bn(BM, EPI)>;
@@ -462,7 +463,16 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     // the epilogue's exchange area (fp8 amax, int8 row maxima) follows this class's ring
     int *scratch = reinterpret_cast<int *>(smem + GSTAGES * STAGE_BYTES);
-    auto tile_end = [&](int e) { return gtab->template end<CLS>(e); };
+    // half0 >= 0 (CLS_128M): the 256-row tiles from index half0 on, each as two tiles of 128 rows
+    constexpr bool CAN_HALVE = CLS == CLS_128M && ROLE == SYNC_NONE;
+    const bool halves = CAN_HALVE && half0 >= 0;
+    auto tile_end = [&](int e) {
+        if constexpr (CAN_HALVE) {
+            if (halves)
+                return gtab->template end<CLS_256>(e);
+        }
+        return gtab->template end<CLS>(e);
+    };
     auto tile_prefix = [&](int e) { return e > 0 ? tile_end(e - 1) : 0; };
     auto row_off = [&](int e) { return e > 0 ? gtab->row_end[e - 1] : 0; };
 
@@ -495,7 +505,9 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     const int nk = (int)(kbytes / GKB);
     const int half_n = p.N / 2;                    // I for SwiGLU
     const int ntn = SWIGLU ? half_n / 128 : p.N / TBN;
-    const int total = __builtin_amdgcn_readfirstlane(tile_prefix(p.L)) * ntn;
+    int total = __builtin_amdgcn_readfirstlane(tile_prefix(p.L)) * ntn;
+    if (halves)
+        total = 2 * (total - half0);
 
     const int G = gridDim.x, logical = first;
     // tiles from the queue tq, in the 8-wave chained kernel: the consumer's heavy tiles (a queue per XCD) and the
@@ -520,7 +532,8 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         int active;    // some row of this wave lies inside the segment (an int: a bool tail makes struct copies go through scratch)
         int nt;        // the expert's only M-tile (W_BY_TILE)
     };
-    auto setup = [&](int tile, Ctx &c) {
+    auto setup = [&](int index, Ctx &c) {
+        const int tile = halves ? half0 + (index >> 1) : index;
         const int lane = lane_here<FRESH>(), band_row = lane >> 3;
         auto chunk_off = [&](int r) { return (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4); };
         int lo = 0, hi = p.L - 1;
@@ -544,7 +557,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         const int nt = rem / gm, mt = grp * GM + rem % gm;
         const int seg0 = __builtin_amdgcn_readfirstlane(row_off(e));
         c.seg1 = min(__builtin_amdgcn_readfirstlane(gtab->row_end[e]), p.M);  // never write past row M
-        c.row0 = seg0 + mt * GBM;
+        c.row0 = halves ? seg0 + mt * 2 * GBM + (index & 1) * GBM : seg0 + mt * GBM;
         c.n0 = SWIGLU ? nt * 128 : nt * TBN;  // first h-column (SwiGLU) or W row (plain)
         // a wave whose rows all lie past the segment skips its MFMAs (it still moves its share of the
         // DMA and meets every barrier): a tile of a short segment costs little more than its weights
@@ -1649,17 +1662,22 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         ge = ROLE == SYNC_PRODUCE && n1 + n2 + n3 >= G ? G : blocks_for(n1 + n2 + n3);
     int nfree = ge, rank = place_among(ge);
     bool is_free = rank < ge;
-    if (n0 > 0 && n0 < G && (G & 7) == 0) {
+    // Without light tiles to fill it, a last round of heavy tiles that would leave half of the blocks idle runs them as
+    // two 128-row tiles each, which end after 0.6 to 0.7 of a heavy tile's time (a k-step alone on its CU: fp8 0.78
+    // against 1.25 us, bf16 0.70 against 1.03 us; 128 heavy tiles alone, K = 7168: fp8 71 against 95 us, int8 62 against
+    // 82 us, bf16 120 against 145 us; 640, K = 4096: 177 against 193, 158 against 167, 280 against 291 us).
+    const int r = n0 % G;
+    const bool halve = ROLE == SYNC_NONE && r > 0 && 2 * r <= G && n1 + n2 + n3 == 0;
+    int hs = pos, hn = halve ? n0 / G : max(0, (n0 - pos + G - 1) / G);  // this block's heavy tiles
+    if (!halve && n0 > 0 && n0 < G && (G & 7) == 0) {
         // Fewer heavy tiles than blocks.  They are split evenly over the 8 XCDs (XCD x takes the run
         // [x hx, (x + 1) hx), consecutive tiles sharing that XCD's L2), so each XCD keeps some blocks free.
         const int xcd = bid & 7, slot = bid >> 3, S = G >> 3;
         const int hx = (n0 + 7) / 8;
         auto heavy_in = [&](int x) { return max(0, min(hx, n0 - x * hx)); };
         const int len = heavy_in(xcd);
-        if (slot < len) {
-            gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, G_NOWHERE, xcd * hx + slot, (len - slot + S - 1) / S, S, wv);
-            lds_sync();  // every wave is done with the first class's ring
-        }
+        hs = xcd * hx + slot;
+        hn = slot < len ? 1 : 0;
         int free_before = 0, busy_before = 0;
         nfree = 0;
         for (int x = 0; x < 8; ++x) {
@@ -1670,14 +1688,15 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         }
         is_free = slot >= len;
         rank = is_free ? free_before + slot - len : busy_before + slot;
-    } else if (n0 > 0) {
+    } else if (!halve && n0 > 0) {
         // At least as many heavy tiles as blocks: round-robin, so the first n0 % G blocks run one more than the rest
-        gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, pos, 0, 0, 1, wv);
-        lds_sync();
-        const int r = n0 % G;
         nfree = G - r;
         is_free = pos >= r;
         rank = is_free ? pos - r : pos;
+    }
+    if (n0 > 0) {
+        gmm_body<DT, EPI, CLS_256, ROLE>(p, gt, G_NOWHERE, hs, __builtin_amdgcn_readfirstlane(hn), G, wv);
+        lds_sync();  // every wave is done with the first class's ring
     }
     if constexpr (ROLE == SYNC_PRODUCE) {
         // the light tiles through one queue; the free blocks start at their own place in it
@@ -1711,9 +1730,11 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         busy_end = __builtin_amdgcn_readfirstlane(busy_end);
     };
     int rs, rn;
-    if (n1 > 0) {
+    if (n1 > 0 || halve) {
         light(n1, 14, rs, rn);
-        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+        if (halve)
+            rs = place_among(blocks_for(2 * r)), rn = 1;
+        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv, TileQueue{}, halve ? n0 - r : -1);
         lds_sync();
     }
     if constexpr (DT == DT_INT8) {
