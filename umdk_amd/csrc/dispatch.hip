@@ -155,7 +155,9 @@ __global__ __launch_bounds__(DISP_WAVES * 64) void dispatch_int8_kernel(
 // once, where a wave per token walks its destinations in turn, two passes over the row for each (128 tokens of 7168
 // columns, about one routed row each, and a shared expert, smooth scales: 6.1 us against 20 + 8.6 us that way).
 constexpr int DF_THREADS = 256, DF_NIT = 2;  // H <= 7168 <= 2 * 256 * 16
-constexpr int DF_MAX_TK = 4096;              // without smooth scales: up to this many picks (more re-read x too often)
+// Without smooth scales up to this many picks (401 tokens of 1280 columns, 4 local picks each: 5.4 against 6.4 us); the
+// block per destination reads x once per pick, the wave per token once.
+constexpr int DF_MAX_TK = 4096;
 static_assert(DF_NIT * DF_THREADS * 16 >= DISP_NIT * 1024, "a row fits the block");
 __global__ __launch_bounds__(DF_THREADS) void dispatch_int8_dest_kernel(
     const uint16_t *__restrict__ x, const int32_t *__restrict__ topk_idx, const int32_t *__restrict__ send_offset,

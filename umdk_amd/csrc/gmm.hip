@@ -16,9 +16,9 @@
 //     (block_epilogue_per_token_dequant.hpp:338-361).
 //
 // Kernel design (gfx950):
-//   * Output tiles of 256, 128 or 32 rows x 256 W rows (SwiGLU: the gate and up rows of one 128-column
+//   * Output tiles of 256, 128, 64 or 32 rows x 256 W rows (SwiGLU: the gate and up rows of one 128-column
 //     block of h; the decode plain GEMM 128 W rows), picked per expert from its row count (the Tile
-//     struct below); the 128/256-row tiles run 8 waves in a 2 x 4 grid, the 32-row tile 4 waves.  MFMA
+//     struct below); the 128/256-row tiles run 8 waves in a 2 x 4 grid, the 32/64-row tiles 4 waves.  MFMA
 //     16x16: v_mfma_f32_16x16x32_bf16, v_mfma_i32_16x16x64_i8, or v_mfma_scale_f32_16x16x128_f8f6f4 with
 //     unit scales for fp8.
 //   * Operands stream through a ring of LDS stages by direct global->LDS DMA (global_load_lds_dwordx4, or
@@ -218,7 +218,7 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 template <int GTHREADS, int MASK, bool FOUR_WAVES = false>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
                                    ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{},
-                                   int few_tiles = 0)
+                                   int few_ntn = 0)
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
     constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(FOUR_WAVES ? CLS_64 : CLS_128M),
@@ -296,7 +296,7 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
 #pragma unroll
         for (int v = 0; v < NWV; ++v)
             all32 += scratch[2 * NWV + v];
-        few = all32 <= few_tiles;
+        few = all32 * few_ntn <= (int)gridDim.x;
     }
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -1499,8 +1499,22 @@ __device__ __forceinline__ int xcd_position()
 // alone and a handful of tiles spreads over the XCDs.
 __device__ __forceinline__ int blocks_for(int n)
 {
-    const int G = gridDim.x, rounds = max((n + G - 1) / G, 1);
-    return __builtin_amdgcn_readfirstlane((G & 7) ? G : min(G, ((n + rounds - 1) / rounds + 7) / 8 * 8));
+    const int G = gridDim.x;
+    if (G & 7)
+        return G;
+    if (n > G) {  // (each division costs a kernel's start about 0.1 us)
+        const int rounds = (n + G - 1) / G;
+        n = (n + rounds - 1) / rounds;
+    }
+    return __builtin_amdgcn_readfirstlane(min(G, max((n + 7) & ~7, 8)));
+}
+// the block's first tile of a round-robin sequence over ge blocks that has given out n tiles before
+__device__ __forceinline__ int continue_after(int n, int rank, int ge)
+{
+    if (n == 0 || rank >= ge)
+        return rank;
+    const int r = rank - n % ge;
+    return __builtin_amdgcn_readfirstlane(r < 0 ? r + ge : r);
 }
 // this block's place among the first g blocks, XCD by XCD; far past every tile for the others
 constexpr int G_NOWHERE = 0x3fffffff;
@@ -1547,30 +1561,27 @@ template <int DT, int EPI> __global__ __launch_bounds__(256, DT == DT_INT8 ? 1 :
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / small_bn(32, EPI);
     build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(), 0,
-                                                ClassRanges{}, (int)gridDim.x / ntn);
+                                                ClassRanges{}, ntn);
     const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p.L - 1)) * ntn;
     const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn;
     // one round-robin sequence over both classes (a tile of either streams the same weight bytes)
     const int ge = blocks_for(n64 + n32), rank = place_among(ge);
-    auto rounds = [&](int r, int n) { return __builtin_amdgcn_readfirstlane(r < ge ? (n - r + ge - 1) / ge : 0); };
     if (n64 > 0) {
-        gmm_body<DT, EPI, CLS_64, SYNC_NONE, false, policy64(DT)>(p, gt, G_NOWHERE, rank, rounds(rank, n64), ge, wv);
+        gmm_body<DT, EPI, CLS_64, SYNC_NONE, false, policy64(DT)>(p, gt, G_NOWHERE, rank, G_NOWHERE, ge, wv);
         lds_sync();
     }
-    const int r32 = __builtin_amdgcn_readfirstlane(rank < ge ? (rank + ge - n64 % ge) % ge : G_NOWHERE);
-    gmm_body<DT, EPI, CLS_32>(p, gt, G_NOWHERE, r32, rounds(r32, n32), ge, wv);
+    gmm_body<DT, EPI, CLS_32>(p, gt, G_NOWHERE, continue_after(n64, rank, ge), G_NOWHERE, ge, wv);
 }
 
 // Prefill: 8 waves, 128- or 256-row tile picked per launch from the actual rows per touched
 // expert (counts are on the device).  The choice is block-uniform and identical in every block.
 // Experts with at least this many rows take the 256-row tile (when the launch allows it).
 constexpr int G_HEAVY_ROWS = 384;
-// In a launch with heavy experts (fp8 and bf16), the experts with fewer rows than this take the 32-row tile on
-// four of the block's waves: their tiles are a weight stream, and that tile's four-stage ring keeps half as
-// many weight bytes again in flight per CU as the 128-row tile's three stages (measured on config 4's fp8
-// GMM1: such a tile streams its 1.8 MB in 46-58 us against 51-65 us, the GEMM 186 vs 193 us; the int8 GEMM
-// measured 1-2% slower and keeps the 128-row tile).  One 32-row tile per expert: two of them would fetch its
-// weights twice.
+// fp8 and bf16: the experts with fewer rows than this take the 32-row tile on four of the block's waves: their tiles
+// are a weight stream, and that tile's four-stage ring keeps half as many weight bytes again in flight per CU as the
+// 128-row tile's three stages (the int8 layer of 22 touched experts measured 390 us with them against 378 us and keeps
+// the 128-row tile).  One 32-row tile per expert: two of them fetch its weights twice (48 fp8 experts of 36 to 281 rows:
+// 255 us a pass at 33 rows, 272 us at 64).
 #ifndef CAM_GMM_SMALL_ROWS
 #define CAM_GMM_SMALL_ROWS 33
 #endif
@@ -1579,12 +1590,10 @@ constexpr int G_SMALL_ROWS = CAM_GMM_SMALL_ROWS;
 // Between two tile classes the block meets at an LDS-only barrier (lds_sync): both prefill loops have drained
 // their DMAs before the last epilogue, so only the ring's LDS reads must be complete (__syncthreads would also
 // wait for the epilogue's global stores; the next class's first DMAs queue behind those stores either way).
-// Prefill: 8 waves.  With the 256-row tile allowed, the experts holding at least G_HEAVY_ROWS rows run
-// 256-row tiles first, then the rest 128-row tiles -- one launch, the longest tiles first, the tile
-// sequence of each block continuing round-robin from the first class into the second, and (fp8, bf16) from
-// there into a third, the experts with fewer than G_SMALL_ROWS rows on 32-row tiles.  A layer whose
-// load is skewed (a few experts with a thousand rows, many with a handful) gets tall tiles where they
-// halve the operand traffic and short ones where a tall tile would multiply padding.
+// Prefill: 8 waves.  With the 256-row tile allowed, the experts holding at least G_HEAVY_ROWS rows run 256-row tiles
+// first, then the rest 128-row tiles and (fp8, bf16) those with fewer than G_SMALL_ROWS rows 32-row tiles, in one launch,
+// the longest tiles first (big_schedule).  A layer whose load is skewed (a few experts with a thousand rows, many with a
+// handful) gets tall tiles where they halve the operand traffic and short ones where a tall tile would multiply padding.
 // short reductions keep the 128-row tile: the 256-row tile's per-tile ring fill and drain would
 // not amortise over fewer than 16 k-steps (at 16, GMM2 of DeepSeek-V3's shapes: the M = 65536 fp8 GMM2
 // 1.71 vs 1.57 PFLOPS, int8 1.97 vs 1.67 POPS, config 4's fp8 GMM2 116 vs 122 us)
@@ -1668,7 +1677,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     // 82 us, bf16 120 against 145 us; 640, K = 4096: 177 against 193, 158 against 167, 280 against 291 us).
     const int r = n0 % G;
     const bool halve = ROLE == SYNC_NONE && r > 0 && 2 * r <= G && n1 + n2 + n3 == 0;
-    int hs = pos, hn = halve ? n0 / G : max(0, (n0 - pos + G - 1) / G);  // this block's heavy tiles
+    int hs = pos, hn = halve ? n0 / G : G_NOWHERE;  // this block's heavy tiles
     if (!halve && n0 > 0 && n0 < G && (G & 7) == 0) {
         // Fewer heavy tiles than blocks.  They are split evenly over the 8 XCDs (XCD x takes the run
         // [x hx, (x + 1) hx), consecutive tiles sharing that XCD's L2), so each XCD keeps some blocks free.
@@ -1712,7 +1721,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     const int nbusy = ge - nfree, ng = is_free ? nfree : nbusy;
     int busy_end = 20, free_end = 0, at = 0;
     auto light = [&](int n, int cost, int &rs, int &rn) {
-        int nf = 0, nb = 0;  // tiles of the free blocks, of the others
+        int nf = 0, nb = 0, layers = 0, last = 0;  // tiles of the free blocks, of the others; this group's layers
         while (nf + nb < n) {
             const bool f = nfree > 0 && (nbusy == 0 || free_end <= busy_end);
             const int layer = min(n - nf - nb, f ? nfree : nbusy);
@@ -1720,12 +1729,14 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
             nb += f ? 0 : layer;
             free_end += f ? cost : 0;
             busy_end += f ? 0 : cost;
+            layers += f == is_free;
+            last = f == is_free ? layer : last;
         }
-        const int mine = is_free ? nf : nb, r = rank < ng ? (rank - at + ng) % ng : G_NOWHERE;
-        // (divisions leave their results in vector registers: scalar ones, as above)
+        // (only a group's last layer can be partial)
+        const int r = rank >= ng ? G_NOWHERE : rank >= at ? rank - at : rank - at + ng;
         rs = __builtin_amdgcn_readfirstlane((is_free ? 0 : nf) + r);
-        rn = __builtin_amdgcn_readfirstlane(max(0, (mine - r + ng - 1) / max(ng, 1)));
-        at = __builtin_amdgcn_readfirstlane((at + mine) % max(ng, 1));
+        rn = __builtin_amdgcn_readfirstlane(r < last ? layers : r < ng ? max(layers - 1, 0) : 0);
+        at = __builtin_amdgcn_readfirstlane(at + last >= ng ? at + last - ng : at + last);
         free_end = __builtin_amdgcn_readfirstlane(free_end);
         busy_end = __builtin_amdgcn_readfirstlane(busy_end);
     };
@@ -1805,19 +1816,17 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
         const GmmArgs p1 = chain_params()->g1;
         const int ntn = p1.N / 2 / 128;
         build_group_tables<Tile<32>::THREADS, 14, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                                    small_ranges(), 0, ClassRanges{}, G / ntn);
+                                                    small_ranges(), 0, ClassRanges{}, ntn);
         const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p1.L - 1)) * ntn;
         const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p1.L - 1)) * ntn;
         t1 = n64 + n32;
         ge = t1 < G ? blocks_for(t1) : G;  // (few tiles spread over the XCDs)
         const int rank = place_among(ge);
-        auto rounds = [&](int r, int n) { return __builtin_amdgcn_readfirstlane(r < ge ? (n - r + ge - 1) / ge : 0); };
         if (n64 > 0) {
-            gmm_body<DT, EPI1, CLS_64, SYNC_PRODUCE, true, policy64(DT)>(p1, gt, G_NOWHERE, rank, rounds(rank, n64), ge, wv);
+            gmm_body<DT, EPI1, CLS_64, SYNC_PRODUCE, true, policy64(DT)>(p1, gt, G_NOWHERE, rank, G_NOWHERE, ge, wv);
             lds_sync();
         }
-        const int r32 = __builtin_amdgcn_readfirstlane(rank < ge ? (rank + ge - n64 % ge) % ge : G_NOWHERE);
-        gmm_body<DT, EPI1, CLS_32, SYNC_PRODUCE, true>(p1, gt, G_NOWHERE, r32, rounds(r32, n32), ge, wv);
+        gmm_body<DT, EPI1, CLS_32, SYNC_PRODUCE, true>(p1, gt, G_NOWHERE, continue_after(n64, rank, ge), G_NOWHERE, ge, wv);
     }
     lds_sync();
     const GmmArgs p2 = chain_params()->g2;
@@ -1831,16 +1840,17 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     const int m32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p2.L - 1)) * (p2.N / BN2);
     // (never more than spreads GMM2's tiles over the free blocks: with few tiles a run would leave most of them idle;
     // one token through 2 of 8 bf16 experts, H = 1024: 16 GMM2 tiles on 16 blocks instead of 4)
-    const int R = __builtin_amdgcn_readfirstlane(
-        max(1, min((GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K),
-                   nfree ? (m64 + m32 + nfree - 1) / nfree : 1)));
+    int R = max(1, (GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K));
+    if (R > 1 && R * nfree > m64 + m32)
+        R = max(1, (m64 + m32 + nfree - 1) / max(nfree, 1));
+    R = __builtin_amdgcn_readfirstlane(R);
     // the block's tiles of both classes in turn: the run [run, run + rn), then next, next + G, ...
     const int run = is_free ? fr * R : 0, rn = is_free ? R : 0, next = R * nfree + pos;
     if (m64 > 0) {
         gmm_body<DT, EPI_PLAIN, CLS_64, SYNC_CONSUME, true, policy64(DT)>(p2, gt, next, run, min(rn, max(m64 - run, 0)), 1, wv);
         lds_sync();
     }
-    const int skip = max(m64 - run, 0), after = max(m64 - next + G - 1, 0) / G;
+    const int skip = max(m64 - run, 0), after = m64 > next ? (m64 - next + G - 1) / G : 0;
     gmm_body<DT, EPI_PLAIN, CLS_32, SYNC_CONSUME, true>(p2, gt, __builtin_amdgcn_readfirstlane(next + after * G - m64),
                                                         max(run - m64, 0), max(rn - skip, 0), 1, wv);
 }
