@@ -1,5 +1,6 @@
 """The native caller of the C ABI (umdk_amd/_camcall.so) on the CPU: argument conversion, the library's errors, and the
 workspace it asks for.  Nothing launches: every call fails in its validation or in its allocation."""
+import numpy as np
 import pytest
 
 from umdk_amd import _lib
@@ -24,6 +25,21 @@ def test_library_errors_keep_their_type_and_text():
 def test_wrong_arguments_are_type_errors(args):
     with pytest.raises(TypeError):
         raw("camhipMoeRoute", *args)
+
+
+@pytest.mark.parametrize("kind", [np.int64, np.int32, np.uint8, np.array])
+def test_sizes_of_any_integer_type(kind):
+    sizes = [kind(v) for v in (64, 1, 8, 2)]
+    want = _lib.workspace_size("camhipDispatchLayout", 1, 64, 1, 8, 2, None, 1, None, 1)
+    seen = []
+
+    def alloc(n):
+        seen.append(n)
+        raise MemoryError("no room")
+
+    with pytest.raises(MemoryError):
+        raw("camhipDispatchLayout", 16, *sizes, None, 16, None, 16, alloc=alloc)
+    assert seen == [want]
 
 
 def test_every_entry_point_is_there():

@@ -5,7 +5,7 @@
 // chain at T = 1021: 90 and 75 us).
 //
 // name(alloc, workspace, workspace_bytes, stream, *args) -> buffer or None
-//   args: the GetWorkspaceSize arguments (pointers as int or None, sizes as int), without the two outputs;
+//   args: the GetWorkspaceSize arguments (pointers as int or None, sizes as any integer), without the two outputs;
 //   alloc: called with the workspace size when it is not 0, returns a tensor (its data_ptr is used and the tensor is
 //          returned); None: the caller's workspace is used;
 //   a failed call raises the exception set by set_error with the library's message.
@@ -35,11 +35,8 @@ template <typename A> bool convert(PyObject *o, A &out)
         }
         out = (A)PyLong_AsVoidPtr(o);
     } else {
-        if (!PyLong_Check(o)) {
-            PyErr_SetString(PyExc_TypeError, "a size argument must be an int");
-            return false;
-        }
-        out = (A)PyLong_AsLongLong(o);
+        // any integer type, numpy's among them, through __index__ (a float has none: TypeError); taken modulo 2^64
+        out = (A)PyLong_AsUnsignedLongLongMask(o);
     }
     return !PyErr_Occurred();
 }
