@@ -217,8 +217,7 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // MASK: the classes the kernel has (the others cost the scan nothing).
 template <int GTHREADS, int MASK, bool FOUR_WAVES = false>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
-                                   ClassRanges cr, int heavy_rows = 0, ClassRanges cr_heavy = ClassRanges{},
-                                   int few_ntn = 0)
+                                   const ClassRanges &cr, int few_ntn = 0)
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
     constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(FOUR_WAVES ? CLS_64 : CLS_128M),
@@ -238,24 +237,6 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
                 v[k] += (c >= cr.lo[k] && c < cr.hi[k]) ? (c + BMS[k] - 1) / BMS[k] : 0;
         v[G_NCLASS] += c;
     };
-    if (heavy_rows > 0) {  // cr_heavy where some expert holds that many rows
-        bool any = false;
-#pragma unroll
-        for (int q = 0; q < PER; ++q)
-            any |= rows[q] >= heavy_rows;
-        int *flag = scratch + NQ * NWV;
-        if (lane == 0)
-            flag[wv] = 0;
-        if (any)
-            flag[wv] = 1;
-        __syncthreads();
-        int f = 0;
-#pragma unroll
-        for (int v = 0; v < NWV; ++v)
-            f |= flag[v];
-        if (f)
-            cr = cr_heavy;
-    }
 #pragma unroll
     for (int q = 0; q < PER; ++q)
         add(rows[q], cnt);
@@ -440,10 +421,11 @@ struct TileQueue {
 // each: the 8-wave kernels have no registers for that).  An expert that fits one M-tile has its weights read exactly
 // once; the M-tiles of an expert of several, which the tile order runs side by side on one XCD, re-read them from that
 // XCD's L2 (48 experts of 36 to 281 rows, fp8, K = 4096, N = 2816: 173 us cached, 205 us nontemporal).  A stream past
-// the caches pays where it spares the L2 lines that others re-read: the 4-wave decode tiles, and the single M-tiles
-// beside heavy experts (the int8 layer of 22 touched experts, one of 2311 rows: 382 us nontemporal, 405 us cached);
-// without heavy experts cached weights are as fast with many tiles (160 against 158 us for 48 experts of 100 rows) and
-// faster with few (54 against 60 us for one expert of 128 rows, N = 4096, K = 7168).
+// the caches pays where it spares the lines that others re-read: the 4-wave decode tiles, and int8's single M-tiles,
+// beside heavy experts (the layer of 22 touched experts, one of 2311 rows: 382 us nontemporal, 405 us cached) and
+// without (weights that differ from call to call: the layer of 8 experts of 1 to 24 rows, H = 2304, I = 1792, 55.3
+// against 59.9 us cached; 16 experts of 2 to 194 rows, H = 4864, I = 512, 86.9 against 90.8 us).  fp8 and bf16 keep
+// their single M-tiles of more than 32 rows cached (48 experts of 100 rows: 160 against 158 us; a class less).
 enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
 constexpr int policy64(int dt) { return dt == DT_FP8 ? W_STREAM : W_BY_TILE; }  // (fp8: no registers for two loops)
 constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? W_STREAM : W_CACHED; }
@@ -1540,7 +1522,7 @@ constexpr size_t G_LDS_BIG_BYTES =
     sizeof(GroupTables);
 static_assert(G_LDS_SMALL_BYTES <= 163840 && G_LDS_BIG_BYTES <= 163840, "LDS budget of a gfx950 workgroup");
 // the table scan's per-wave totals (before any ring use)
-static_assert(sizeof(int) * (G_NCLASS + 2) * (GMAX_THREADS / 64) <= ring_bytes<32, 128>(), "table-scan scratch");
+static_assert(sizeof(int) * (G_NCLASS + 1) * (GMAX_THREADS / 64) <= ring_bytes<32, 128>(), "table-scan scratch");
 
 // Decode-sized segments (4 waves): 32-row tiles, and 64-row tiles for the experts of more rows (64 bf16 experts of 37
 // rows on average, H = 2048, I = 1408: the decode step 245 us against 282 us with two 32-row tiles, each streaming the
@@ -1560,8 +1542,8 @@ template <int DT, int EPI> __global__ __launch_bounds__(256, DT == DT_INT8 ? 1 :
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / small_bn(32, EPI);
-    build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(), 0,
-                                                ClassRanges{}, ntn);
+    build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(),
+                                                ntn);
     const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p.L - 1)) * ntn;
     const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn;
     // one round-robin sequence over both classes (a tile of either streams the same weight bytes)
@@ -1601,14 +1583,13 @@ __host__ __device__ constexpr bool big_tall(int allow256, int K, int dt)
 {
     return allow256 && (int)((uint32_t)K * (dt == DT_BF16 ? 2 : 1) / GKB) >= CAM_GMM_MIN_NK256;
 }
-// heavy: the launch has experts for 256-row tiles; int8: the single 128-row tiles beside them are a class of their
-// own (fp8 and bf16 move their smallest experts to 32-row tiles instead, and one GEMM loop fewer in their kernels leaves
-// the 256-row loop more registers: 157 against 238 spilled scalars in the fp8 GMM1)
-template <int DT> __device__ __forceinline__ ClassRanges big_ranges(bool tall, bool heavy)
+// int8: the single 128-row tiles are a class of their own (fp8 and bf16 move their smallest experts to 32-row tiles
+// instead: one GEMM loop fewer in their kernels leaves the 256-row loop more registers)
+template <int DT> __device__ __forceinline__ ClassRanges big_ranges(bool tall)
 {
     constexpr int SMALL = DT == DT_INT8 ? 1 : G_SMALL_ROWS;  // rows below: the 32-row tile class
     const int top = tall ? G_HEAVY_ROWS : 0x7fffffff, small = tall ? SMALL : 1;
-    const int multi = heavy && DT == DT_INT8 ? 129 : small;
+    const int multi = tall && DT == DT_INT8 ? 129 : small;
     return ClassRanges{{top, multi, small, 1}, {0x7fffffff, top, multi, small}};
 }
 
@@ -1772,8 +1753,7 @@ template <int DT, int EPI> __global__ __launch_bounds__(512, 1) void gmm_kernel_
     const bool tall = big_tall(p.allow256, p.K, DT);
     // every class's expert table, from one read of the counts
     build_group_tables<GMAX_THREADS, DT == DT_INT8 ? 7 : 11>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem),
-                                     big_ranges<DT>(tall, false),
-                                     DT == DT_INT8 && tall ? G_HEAVY_ROWS : 0, big_ranges<DT>(tall, true));
+                                     big_ranges<DT>(tall));
     big_schedule<DT, EPI, SYNC_NONE>(p, gt, wv);
 }
 
@@ -1793,7 +1773,7 @@ template <int DT, int EPI1> __global__ __launch_bounds__(512, 1) void gmm_chain_
         const GmmArgs p1 = chain_params()->g1;
         tall = big_tall(p1.allow256, p1.K, DT);  // the host checked that GMM2 makes the same choice
         build_group_tables<GMAX_THREADS, 11>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                         big_ranges<DT>(tall, false));
+                                         big_ranges<DT>(tall));
         big_schedule<DT, EPI1, SYNC_PRODUCE>(p1, gt, wv);
     }
     lds_sync();  // every wave is done with GMM1's last ring
@@ -1816,7 +1796,7 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
         const GmmArgs p1 = chain_params()->g1;
         const int ntn = p1.N / 2 / 128;
         build_group_tables<Tile<32>::THREADS, 14, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                                    small_ranges(), 0, ClassRanges{}, ntn);
+                                                    small_ranges(), ntn);
         const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p1.L - 1)) * ntn;
         const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p1.L - 1)) * ntn;
         t1 = n64 + n32;
