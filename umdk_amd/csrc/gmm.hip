@@ -427,7 +427,10 @@ struct TileQueue {
 // against 59.9 us cached; 16 experts of 2 to 194 rows, H = 4864, I = 512, 86.9 against 90.8 us).  fp8 and bf16 keep
 // their single M-tiles of more than 32 rows cached (48 experts of 100 rows: 160 against 158 us; a class less).
 enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
-constexpr int policy64(int dt) { return dt == DT_FP8 ? W_STREAM : W_BY_TILE; }  // (fp8: no registers for two loops)
+// 64-row tiles in fp8, which has no registers for two loops: as a stream, also where an expert has several (the decode
+// step of 400 tokens, 64 experts, H = 2048, I = 1408 140 against 148 us cached; 32 experts of 44 rows, H = 4096,
+// I = 1536: 144 against 148 us; the steps of 16 to 4096 tokens with a shared expert on all of them within 1%).
+constexpr int policy64(int dt) { return dt == DT_FP8 ? W_STREAM : W_BY_TILE; }
 constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? W_STREAM : W_CACHED; }
 
 template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS)>
@@ -1254,7 +1257,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
 
             if constexpr (FP8) {
                 // One K=128 MFMA per fragment pair and k-step, and each is one scale block, so its result
-                // is scaled on the VALU.  W fragments are double-buffered; A fragments are refilled row by
+                // is scaled on the VALU.  W fragments are double-buffered (but see ONE_W); A fragments are refilled row by
                 // row right after the row's MFMAs have issued (one register set plus one W set in flight).
                 // The scaling lags one fragment row behind (row i-1's results are scaled while row i's MFMAs
                 // issue, 4 VALU : 1 MFMA), so the MFMA pipe never waits for a result it has just produced.
@@ -1328,6 +1331,11 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
                         rd_a(i, ks_next);
                     }
                 };
+                // (64-row tile: one W set, refilled behind the MFMAs that use it.  Beside 64 accumulators the second set
+                // spilled, in the chained launch 19 registers that its 32-row loop reloaded too, and a weight stream
+                // does not wait for those reads: the decode steps of 400 tokens, 64 experts, H = 2048, I = 1408 151 ->
+                // 140 us, of 64 tokens, 32 of 256 experts and a shared one, H = 7168, I = 2048 249 -> 221 us)
+                constexpr bool ONE_W = CLS == CLS_64;
                 WRegs w0, w1;
 #pragma unroll
                 for (int i = 0; i < IF; ++i)
@@ -1335,6 +1343,14 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
                 rd_w(w0, 0);
                 auto kloop = [&](auto act, auto nt) {
                     int ks = 0;
+                    if constexpr (ONE_W) {
+                        for (; ks < nk; ++ks) {
+                            step_edge();
+                            mm(w0, ks + 1, act, nt);
+                            rd_w(w0, ks + 1);
+                        }
+                        return;
+                    }
                     for (; ks + 1 < nk; ks += 2) {
                         step_edge();
                         rd_w(w1, ks + 1);
