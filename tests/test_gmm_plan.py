@@ -1,0 +1,42 @@
+"""The rules that give a decode GEMM launch's tiles to its blocks (umdk_amd/csrc/gmm_plan.h), compiled for the host."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "umdk_amd", "csrc")
+SOURCE = """
+#include "gmm_plan.h"
+extern "C" int rows32(int n32, int n64, int G) { return cam::small_rows32(n32, n64, G); }
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    (d / "plan.cpp").write_text(SOURCE)
+    so = str(d / "plan.so")
+    subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, str(d / "plan.cpp"), "-o", so],
+                   check=True)
+    return ctypes.CDLL(so)
+
+
+def tiles(counts, ntn):
+    """32-row tiles of a GEMM with ntn N-tiles, and its tiles with 64-row ones for the experts of more than 32 rows."""
+    return (sum(-(-c // 32) for c in counts) * ntn,
+            sum(-(-c // 64) if c > 32 else -(-c // 32) for c in counts) * ntn)
+
+
+def test_64_row_tiles_only_where_they_save_rounds(plan):
+    ragged = [20, 36, 62, 40, 66, 33, 40, 34, 15, 14, 53, 45, 22, 33, 28, 14]
+    n32, n64 = tiles(ragged, 18)  # 486 and 306 tiles on 256 blocks: two rounds either way
+    assert -(-n32 // 256) == -(-n64 // 256) == 2 and plan.rows32(n32, n64, 256)
+    assert not plan.rows32(*tiles([45] * 16, 32), 256)   # 1024 -> 512 tiles
+    assert not plan.rows32(*tiles([47] * 8, 56), 256)    # 896 -> 448
+    assert plan.rows32(*tiles([45] * 8, 16), 256)        # one round
+    assert plan.rows32(*tiles([20] * 64, 56), 256)       # no expert of more than 32 rows
+    for n32 in range(1, 3000, 7):  # never more rounds, weighted by a 64-row tile's time
+        for n64 in range(max(1, n32 // 2), n32 + 1, 13):
+            if not plan.rows32(n32, n64, 256):
+                assert 1.25 * -(-n64 // 256) <= -(-n32 // 256)

@@ -8,6 +8,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from test_gmm_plan import plan, tiles  # noqa: F401 (plan is a fixture)
 from test_gpu_chain import DT_BF16, DT_FP8, Case, lib  # noqa: F401 (lib is a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -71,12 +72,12 @@ def rows_to(c, cap):
 
 @pytest.mark.parametrize("dt", [DT_FP8, DT_BF16])
 @pytest.mark.parametrize("counts,H,I", BOTH)
-def test_decode_tiles_of_both_heights(lib, counts, H, I, dt):  # noqa: F811
+def test_decode_tiles_of_both_heights(lib, plan, counts, H, I, dt):  # noqa: F811
     # against the same groups at a prefill capacity: the 8-wave kernels, every sum in the same order
     print(f"decode tiles of both heights counts={counts[:5]}.. dt={dt}", flush=True)
     c = Case(counts, H, I, dt, 90)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert c.cap <= 48 * c.L and sum(-(-n // 32) for n in counts) * (I // 128) > cus
+    assert c.cap <= 48 * c.L and not plan.rows32(*tiles(counts, I // 128), cus) and min(n for n in counts if n) <= 32
     b = rows_to(c, 48 * c.L + 1)
     for _ in range(2):
         c.new_outputs()

@@ -49,6 +49,7 @@
 
 #include "cam_device.h"
 #include "gmm.h"
+#include "gmm_plan.h"
 #include "launchers.h"
 
 namespace cam {
@@ -116,7 +117,8 @@ constexpr int class_bm(int cls) { return cls == CLS_256 ? 256 : cls == CLS_32 ? 
 // Expert tables of a launch, built once at kernel start: per tile class the inclusive prefix of M-tiles per
 // expert, and the inclusive prefix of rows per expert (the exclusive prefix of expert e is entry e-1, or 0 for
 // e = 0; no entry for it keeps the tables within the LDS budget).  The last two classes share a word: at most one
-// tile per expert in either (<= 512), or few tiles in all (see small_ranges).
+// tile per expert in either (<= 512); in a 4-wave launch (at most 48 rows per expert on average) CLS_32 alone, at most
+// M / 32 + L tiles.
 struct GroupTables {
     int tile_end[G_NCLASS - 2][G_MAX_L];
     uint32_t tile_end_s[G_MAX_L];  // CLS_128S << 16 | CLS_32
@@ -214,10 +216,10 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // the counts.  Only experts with a row count in a class's [lo, hi) get tiles of that class (a launch may
 // split the experts between tile heights); the row offsets count every expert (they locate segments in
 // dispatch order).
-// MASK: the classes the kernel has (the others cost the scan nothing).
+// MASK: the classes the kernel has (the others cost the scan nothing).  ntn (FOUR_WAVES): the GEMM's N-tiles.
 template <int GTHREADS, int MASK, bool FOUR_WAVES = false>
 __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
-                                   const ClassRanges &cr, int few_ntn = 0)
+                                   const ClassRanges &cr, int ntn = 0)
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
     constexpr int BMS[G_NCLASS] = {class_bm(0), class_bm(FOUR_WAVES ? CLS_64 : CLS_128M),
@@ -271,13 +273,17 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
             ex += used(k) && v < wv ? scratch[k * NWV + v] : 0;
         run[k] = ex;
     }
-    bool few = false;
+    bool rows32 = false;
     if constexpr (FOUR_WAVES) {  // slot 2 counts the M-tiles with 32-row tiles throughout (small_ranges)
-        int all32 = 0;
+        int n[G_NCLASS] = {};
 #pragma unroll
-        for (int v = 0; v < NWV; ++v)
-            all32 += scratch[2 * NWV + v];
-        few = all32 * few_ntn <= (int)gridDim.x;
+        for (int k = 1; k < G_NCLASS; ++k) {
+#pragma unroll
+            for (int v = 0; v < NWV; ++v)
+                n[k] += scratch[k * NWV + v];
+            n[k] = __builtin_amdgcn_readfirstlane(n[k]) * ntn;
+        }
+        rows32 = small_rows32(n[2], n[CLS_128M] + n[CLS_32], (int)gridDim.x);
     }
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -286,8 +292,8 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
         if (e < L) {
             if constexpr (FOUR_WAVES) {
                 gt.tile_end[CLS_256][e] = 0;
-                gt.tile_end[CLS_128M][e] = few ? 0 : run[CLS_128M];
-                gt.tile_end_s[e] = (uint32_t)(few ? run[2] : run[CLS_32]);
+                gt.tile_end[CLS_128M][e] = rows32 ? 0 : run[CLS_128M];
+                gt.tile_end_s[e] = (uint32_t)(rows32 ? run[2] : run[CLS_32]);
                 gt.row_end[e] = run[G_NCLASS];
                 continue;
             }
@@ -1545,8 +1551,8 @@ static_assert(sizeof(int) * (G_NCLASS + 1) * (GMAX_THREADS / 64) <= ring_bytes<3
 // expert's weights).  fp8 and bf16 are bounded to two waves per SIMD although the LDS allows one: with up to
 // 512 registers a wave the compiler keeps operands in accumulation registers and moves 24 to 64 of them per k-step (the
 // int8 GMM2 alone measured faster that way, 76 against 78 us).
-// With no more 32-row tiles than blocks they all run at once, and two of them end before one 64-row tile does (32 fp8
-// experts of 15 rows, K = 5888, two N-tiles each: GMM1 and GMM2 75 us against 78 us): 32-row tiles throughout then.
+// Where the 64-row tiles do not save rounds of tiles, 32-row tiles run throughout (small_rows32; with no more of them than
+// blocks they all run at once: 32 fp8 experts of 15 rows, K = 5888, two N-tiles each: GMM1 and GMM2 75 us against 78 us).
 constexpr int G_ROWS32 = 32;
 __device__ __forceinline__ ClassRanges small_ranges()
 {
