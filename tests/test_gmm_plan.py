@@ -9,6 +9,12 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = """
 #include "gmm_plan.h"
 extern "C" int rows32(int n32, int n64, int G) { return cam::small_rows32(n32, n64, G); }
+extern "C" int blocks(int n, int G) { return cam::plan_blocks(n, G); }
+extern "C" void gmm2(int b, int G, int t1, int ge, int t2, int c1, int c2, int *out)
+{
+    const cam::ChainGmm2 p = cam::plan_chain_gmm2(b, G, t1, ge, t2, c1, c2);
+    out[0] = p.run, out[1] = p.rn, out[2] = p.next;
+}
 """
 
 
@@ -40,3 +46,22 @@ def test_64_row_tiles_only_where_they_save_rounds(plan):
         for n64 in range(max(1, n32 // 2), n32 + 1, 13):
             if not plan.rows32(n32, n64, 256):
                 assert 1.25 * -(-n64 // 256) <= -(-n32 // 256)
+
+
+@pytest.mark.parametrize("G", [256, 304, 250])
+@pytest.mark.parametrize("t1,t2,c1,c2", [(192, 432, 2304, 512), (200, 1024, 4096, 768), (255, 256, 1024, 512),
+                                         (256, 900, 2048, 1024), (8, 16, 1024, 256), (1, 1, 7168, 1024), (0, 0, 512, 512),
+                                         (330, 700, 2048, 704), (700, 2000, 14336, 1024), (1144, 2300, 512, 4096)])
+def test_chained_decode_gmm2_tiles(plan, G, t1, t2, c1, c2):
+    ge = plan.blocks(t1, G) if t1 < G else G
+    out, seen, per_block = (ctypes.c_int * 3)(), [], []
+    for b in range(G):
+        plan.gmm2(b, G, t1, ge, t2, c1, c2, out)
+        run, rn, nxt = out
+        mine = [t for t in list(range(run, run + rn)) + list(range(nxt, t2, G)) if t < t2]
+        assert mine == sorted(mine)  # the first index past the tiles ends a block's sequence
+        seen += mine
+        per_block.append(len(mine))
+    assert sorted(seen) == list(range(t2))  # every tile once
+    if t1 <= G:  # no block may start GMM2 before the others: even shares
+        assert max(per_block) <= -(-t2 // G)

@@ -1490,27 +1490,9 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     }
 }
 
-// XCD-aware order: blocks b, b+8, b+16, ... run on the same XCD; give them consecutive positions,
-// so that a run of consecutive tiles shares that XCD's L2
-__device__ __forceinline__ int xcd_position()
-{
-    const int G = gridDim.x;
-    return (G & 7) ? (int)blockIdx.x : (int)((blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3));
-}
-
-// Blocks that share n equal tiles in whole rounds: with R = ceil(n / G) rounds, only the first ceil(n / R) blocks
-// (rounded up to whole XCDs) take tiles, R each at most, so a last partial round does not leave a few blocks streaming
-// alone and a handful of tiles spreads over the XCDs.
 __device__ __forceinline__ int blocks_for(int n)
 {
-    const int G = gridDim.x;
-    if (G & 7)
-        return G;
-    if (n > G) {  // (each division costs a kernel's start about 0.1 us)
-        const int rounds = (n + G - 1) / G;
-        n = (n + rounds - 1) / rounds;
-    }
-    return __builtin_amdgcn_readfirstlane(min(G, max((n + 7) & ~7, 8)));
+    return __builtin_amdgcn_readfirstlane(plan_blocks(n, (int)gridDim.x));
 }
 // the block's first tile of a round-robin sequence over ge blocks that has given out n tiles before
 __device__ __forceinline__ int continue_after(int n, int rank, int ge)
@@ -1520,13 +1502,7 @@ __device__ __forceinline__ int continue_after(int n, int rank, int ge)
     const int r = rank - n % ge;
     return __builtin_amdgcn_readfirstlane(r < 0 ? r + ge : r);
 }
-// this block's place among the first g blocks, XCD by XCD; far past every tile for the others
-constexpr int G_NOWHERE = 0x3fffffff;
-__device__ __forceinline__ int place_among(int g)
-{
-    const int b = blockIdx.x;
-    return (gridDim.x & 7) ? b : b < g ? (b & 7) * (g >> 3) + (b >> 3) : G_NOWHERE;
-}
+__device__ __forceinline__ int place_among(int g) { return plan_place((int)blockIdx.x, g, (int)gridDim.x); }
 
 // LDS of a launch: a class's ring of stages, then that class's epilogue exchange area; the expert tables
 // sit at the end of the launch's LDS (the same place for every class of a launch).
@@ -1808,10 +1784,9 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     // Decode tiles are weight streams of fixed size, so the two phases are balanced statically: GMM1's tiles go
-    // round-robin over every block, and the blocks left with one GMM1 tile fewer start GMM2 with a run of R
-    // tiles, R = a GMM1 tile's weight bytes over a GMM2 tile's (256 rows of K1 against 128 rows of K2).  Those
-    // first GMM2 tiles (the first experts) depend only on GMM1's first round.
-    const int pos = xcd_position(), G = gridDim.x;
+    // round-robin over every block, GMM2's as plan_chain_gmm2 says.  A run's GMM2 tiles (the first experts) depend
+    // only on GMM1's first rounds.
+    const int G = gridDim.x;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int t1, ge;
     {
@@ -1832,22 +1807,13 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     }
     lds_sync();
     const GmmArgs p2 = chain_params()->g2;
-    // the blocks with one GMM1 tile fewer: nfree, this one number fr of them
-    const bool few = ge < G;
-    const int r1 = few ? ge : t1 % G, nfree = r1 ? G - r1 : 0;
-    const int fr = (few ? (int)blockIdx.x : pos) - r1;
-    const bool is_free = nfree > 0 && fr >= 0;
     constexpr int BN2 = small_bn(32, EPI_PLAIN);
     const int m64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p2.L - 1)) * (p2.N / BN2);
     const int m32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p2.L - 1)) * (p2.N / BN2);
-    // (never more than spreads GMM2's tiles over the free blocks: with few tiles a run would leave most of them idle;
-    // one token through 2 of 8 bf16 experts, H = 1024: 16 GMM2 tiles on 16 blocks instead of 4)
-    int R = max(1, (GBN * chain_params()->g1.K + BN2 * p2.K / 2) / (BN2 * p2.K));
-    if (R > 1 && R * nfree > m64 + m32)
-        R = max(1, (m64 + m32 + nfree - 1) / max(nfree, 1));
-    R = __builtin_amdgcn_readfirstlane(R);
     // the block's tiles of both classes in turn: the run [run, run + rn), then next, next + G, ...
-    const int run = is_free ? fr * R : 0, rn = is_free ? R : 0, next = R * nfree + pos;
+    const ChainGmm2 g2 = plan_chain_gmm2((int)blockIdx.x, G, t1, ge, m64 + m32, GBN * chain_params()->g1.K, BN2 * p2.K);
+    const int run = __builtin_amdgcn_readfirstlane(g2.run), rn = __builtin_amdgcn_readfirstlane(g2.rn);
+    const int next = __builtin_amdgcn_readfirstlane(g2.next);
     if (m64 > 0) {
         gmm_body<DT, EPI_PLAIN, CLS_64, SYNC_CONSUME, true, policy64(DT)>(p2, gt, next, run, min(rn, max(m64 - run, 0)), 1, wv);
         lds_sync();
