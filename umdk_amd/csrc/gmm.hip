@@ -217,8 +217,12 @@ __device__ uint64_t g_cam_tl[G_TL_BLOCKS * G_TL_SLOTS][3];
 // split the experts between tile heights); the row offsets count every expert (they locate segments in
 // dispatch order).
 // MASK: the classes the kernel has (the others cost the scan nothing).  ntn (FOUR_WAVES): the GEMM's N-tiles.
+// Returns the M-tiles of each class.
+struct ClassTiles {
+    int n[G_NCLASS];
+};
 template <int GTHREADS, int MASK, bool FOUR_WAVES = false>
-__device__ void build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
+__device__ ClassTiles build_group_tables(const int64_t *__restrict__ group_list, int L, GroupTables &gt, int *scratch,
                                    const ClassRanges &cr, int ntn = 0)
 {
     constexpr int NQ = G_NCLASS + 1;  // tile counts per class, then rows
@@ -264,27 +268,25 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
             scratch[k * NWV + wv] = inc[k];
     }
     __syncthreads();
-    int run[NQ];
+    int run[NQ], tot[NQ];  // the thread's exclusive prefix, the block's totals
+    const int w = __builtin_amdgcn_readfirstlane(wv);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-        int ex = inc[k] - cnt[k];
+        int ex = inc[k] - cnt[k], all = 0;
+        if (used(k)) {
 #pragma unroll
-        for (int v = 0; v < NWV; ++v)
-            ex += used(k) && v < wv ? scratch[k * NWV + v] : 0;
+            for (int v = 0; v < NWV; ++v) {
+                const int n = scratch[k * NWV + v];
+                ex += v < w ? n : 0;
+                all += n;
+            }
+        }
         run[k] = ex;
+        tot[k] = __builtin_amdgcn_readfirstlane(all);
     }
     bool rows32 = false;
-    if constexpr (FOUR_WAVES) {  // slot 2 counts the M-tiles with 32-row tiles throughout (small_ranges)
-        int n[G_NCLASS] = {};
-#pragma unroll
-        for (int k = 1; k < G_NCLASS; ++k) {
-#pragma unroll
-            for (int v = 0; v < NWV; ++v)
-                n[k] += scratch[k * NWV + v];
-            n[k] = __builtin_amdgcn_readfirstlane(n[k]) * ntn;
-        }
-        rows32 = small_rows32(n[2], n[CLS_128M] + n[CLS_32], (int)gridDim.x);
-    }
+    if constexpr (FOUR_WAVES)  // slot 2 counts the M-tiles with 32-row tiles throughout (small_ranges)
+        rows32 = small_rows32(tot[2] * ntn, (tot[CLS_128M] + tot[CLS_32]) * ntn, (int)gridDim.x);
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
         const int e = tid * PER + q;
@@ -304,6 +306,9 @@ __device__ void build_group_tables(const int64_t *__restrict__ group_list, int L
         }
     }
     __syncthreads();
+    if constexpr (FOUR_WAVES)
+        return {0, rows32 ? 0 : tot[CLS_128M], 0, rows32 ? tot[2] : tot[CLS_32]};
+    return {tot[CLS_256], tot[CLS_128M], tot[CLS_128S], tot[CLS_32]};
 }
 
 // LDS byte offset of 16-byte chunk `chunk` of row `row`.  Chunks are XOR-swizzled by (row >> 1) & 7:
@@ -1540,10 +1545,9 @@ template <int DT, int EPI> __global__ __launch_bounds__(256, DT == DT_INT8 ? 1 :
     GroupTables *gt = reinterpret_cast<GroupTables *>(smem + G_LDS_SMALL_BYTES - sizeof(GroupTables));
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int ntn = EPI != EPI_PLAIN ? p.N / 2 / 128 : p.N / small_bn(32, EPI);
-    build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt, reinterpret_cast<int *>(smem), small_ranges(),
-                                                ntn);
-    const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p.L - 1)) * ntn;
-    const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p.L - 1)) * ntn;
+    const ClassTiles mt = build_group_tables<Tile<32>::THREADS, 14, true>(p.group_list, p.L, *gt,
+                                                                          reinterpret_cast<int *>(smem), small_ranges(), ntn);
+    const int n64 = mt.n[CLS_128M] * ntn, n32 = mt.n[CLS_32] * ntn;
     // one round-robin sequence over both classes (a tile of either streams the same weight bytes)
     const int ge = blocks_for(n64 + n32), rank = place_among(ge);
     if (n64 > 0) {
@@ -1789,13 +1793,13 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     const int G = gridDim.x;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int t1, ge;
+    ClassTiles mt;
     {
         const GmmArgs p1 = chain_params()->g1;
         const int ntn = p1.N / 2 / 128;
-        build_group_tables<Tile<32>::THREADS, 14, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
-                                                    small_ranges(), ntn);
-        const int n64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p1.L - 1)) * ntn;
-        const int n32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p1.L - 1)) * ntn;
+        mt = build_group_tables<Tile<32>::THREADS, 14, true>(p1.group_list, p1.L, *gt, reinterpret_cast<int *>(smem),
+                                                             small_ranges(), ntn);
+        const int n64 = mt.n[CLS_128M] * ntn, n32 = mt.n[CLS_32] * ntn;
         t1 = n64 + n32;
         ge = t1 < G ? blocks_for(t1) : G;  // (few tiles spread over the XCDs)
         const int rank = place_among(ge);
@@ -1808,8 +1812,7 @@ template <int DT, int EPI1> __global__ __launch_bounds__(256, 2) void gmm_chain_
     lds_sync();
     const GmmArgs p2 = chain_params()->g2;
     constexpr int BN2 = small_bn(32, EPI_PLAIN);
-    const int m64 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_64>(p2.L - 1)) * (p2.N / BN2);
-    const int m32 = __builtin_amdgcn_readfirstlane(gt->template end<CLS_32>(p2.L - 1)) * (p2.N / BN2);
+    const int m64 = mt.n[CLS_128M] * (p2.N / BN2), m32 = mt.n[CLS_32] * (p2.N / BN2);
     // the block's tiles of both classes in turn: the run [run, run + rn), then next, next + G, ...
     const ChainGmm2 g2 = plan_chain_gmm2((int)blockIdx.x, G, t1, ge, m64 + m32, GBN * chain_params()->g1.K, BN2 * p2.K);
     const int run = __builtin_amdgcn_readfirstlane(g2.run), rn = __builtin_amdgcn_readfirstlane(g2.rn);
