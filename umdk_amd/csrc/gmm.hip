@@ -444,10 +444,10 @@ enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
 constexpr int policy64(int dt) { return dt == DT_FP8 ? W_STREAM : W_BY_TILE; }
 constexpr int class_policy(int cls) { return cls == CLS_128S || cls == CLS_32 ? W_STREAM : W_CACHED; }
 
-template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS)>
+template <int DT, int EPI, int CLS, int ROLE = SYNC_NONE, bool EAGER = false, int POL = class_policy(CLS), bool HALVES = false>
 __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gtab, int first, int rs = 0, int rn = 0,
                                         int rstride = 1, int wv = -1, const TileQueue &tq = TileQueue{},
-                                        int half0 = -1)
+                                        int half0 = 0)
 {
     constexpr int BM = class_bm(CLS);
     using TC = Tile<BM, small_bn(BM, EPI)>;
@@ -459,16 +459,11 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     // the epilogue's exchange area (fp8 amax, int8 row maxima) follows this class's ring
     int *scratch = reinterpret_cast<int *>(smem + GSTAGES * STAGE_BYTES);
-    // half0 >= 0 (CLS_128M): the 256-row tiles from index half0 on, each as two tiles of 128 rows
-    constexpr bool CAN_HALVE = CLS == CLS_128M && ROLE == SYNC_NONE;
-    const bool halves = CAN_HALVE && half0 >= 0;
-    auto tile_end = [&](int e) {
-        if constexpr (CAN_HALVE) {
-            if (halves)
-                return gtab->template end<CLS_256>(e);
-        }
-        return gtab->template end<CLS>(e);
-    };
+    // HALVES (CLS_128M): the 256-row tiles from index half0 on, each as two tiles of 128 rows.  (An instance of its own: a
+    // run-time choice in the light tiles' one cost them scalar registers, the fp8 GEMMs of 16 experts of 256 rows, H = 7168,
+    // I = 1024 204.6 against 201.0 us, of 8 experts of 856 to 2893 rows, H = 1024, I = 13056 811 against 796 us.)
+    static_assert(!HALVES || CLS == CLS_128M);
+    auto tile_end = [&](int e) { return gtab->template end<HALVES ? CLS_256 : CLS>(e); };
     auto tile_prefix = [&](int e) { return e > 0 ? tile_end(e - 1) : 0; };
     auto row_off = [&](int e) { return e > 0 ? gtab->row_end[e - 1] : 0; };
 
@@ -502,7 +497,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
     const int half_n = p.N / 2;                    // I for SwiGLU
     const int ntn = SWIGLU ? half_n / 128 : p.N / TBN;
     int total = __builtin_amdgcn_readfirstlane(tile_prefix(p.L)) * ntn;
-    if (halves)
+    if (HALVES)
         total = 2 * (total - half0);
 
     const int G = gridDim.x, logical = first;
@@ -529,7 +524,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         int nt;        // the expert's only M-tile (W_BY_TILE)
     };
     auto setup = [&](int index, Ctx &c) {
-        const int tile = halves ? half0 + (index >> 1) : index;
+        const int tile = HALVES ? half0 + (index >> 1) : index;
         const int lane = lane_here<FRESH>(), band_row = lane >> 3;
         auto chunk_off = [&](int r) { return (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4); };
         int lo = 0, hi = p.L - 1;
@@ -553,7 +548,7 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
         const int nt = rem / gm, mt = grp * GM + rem % gm;
         const int seg0 = __builtin_amdgcn_readfirstlane(row_off(e));
         c.seg1 = min(__builtin_amdgcn_readfirstlane(gtab->row_end[e]), p.M);  // never write past row M
-        c.row0 = halves ? seg0 + mt * 2 * GBM + (index & 1) * GBM : seg0 + mt * GBM;
+        c.row0 = HALVES ? seg0 + mt * 2 * GBM + (index & 1) * GBM : seg0 + mt * GBM;
         c.n0 = SWIGLU ? nt * 128 : nt * TBN;  // first h-column (SwiGLU) or W row (plain)
         // a wave whose rows all lie past the segment skips its MFMAs (it still moves its share of the
         // DMA and meets every barrier): a tile of a short segment costs little more than its weights
@@ -1658,7 +1653,7 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
     // two 128-row tiles each, which end after 0.6 to 0.7 of a heavy tile's time (a k-step alone on its CU: fp8 0.78
     // against 1.25 us, bf16 0.70 against 1.03 us; 128 heavy tiles alone, K = 7168: fp8 71 against 95 us, int8 62 against
     // 82 us, bf16 120 against 145 us; 640, K = 4096: 177 against 193, 158 against 167, 280 against 291 us).
-    const int r = n0 % G;
+    const int r = n0 < G ? n0 : n0 % G;
     const bool halve = ROLE == SYNC_NONE && r > 0 && 2 * r <= G && n1 + n2 + n3 == 0;
     int hs = pos, hn = halve ? n0 / G : G_NOWHERE;  // this block's heavy tiles
     if (!halve && n0 > 0 && n0 < G && (G & 7) == 0) {
@@ -1724,11 +1719,16 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         busy_end = __builtin_amdgcn_readfirstlane(busy_end);
     };
     int rs, rn;
-    if (n1 > 0 || halve) {
+    if constexpr (ROLE == SYNC_NONE) {
+        if (halve) {
+            gmm_body<DT, EPI, CLS_128M, ROLE, false, W_CACHED, true>(p, gt, G_NOWHERE, place_among(blocks_for(2 * r)), 1, G, wv,
+                                                                     TileQueue{}, n0 - r);
+            return;
+        }
+    }
+    if (n1 > 0) {
         light(n1, 14, rs, rn);
-        if (halve)
-            rs = place_among(blocks_for(2 * r)), rn = 1;
-        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv, TileQueue{}, halve ? n0 - r : -1);
+        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
         lds_sync();
     }
     if constexpr (DT == DT_INT8) {
