@@ -1008,6 +1008,12 @@ __device__ __forceinline__ int gmm_body(const GmmArgs &p, const GroupTables *gta
                         rd_a(i);
 #pragma unroll
                     for (int i = 0; i < IF; ++i) {
+                        // bf16: the rows stay in this order.  Left to itself the compiler moved reads and waits across
+                        // them, another way in each build (W rows 4096 x 14336, 8 experts of 2000 rows: 1459 us with
+                        // the rows held, 1527, 1543 and 1509 us in three builds without; 28672 x 4096: 2802 against
+                        // 2829 to 2856 us; 4 experts of 4608 rows, K = 5248, N = 2304: 362 against 362 to 373 us)
+                        if constexpr (DT == DT_BF16)
+                            __builtin_amdgcn_sched_barrier(0);
                         if (i + AHEAD < IF)
                             rd_a(i + AHEAD);
                         const float sgi = FP8 ? sa[i] * sg : 0.0f, sui = FP8 ? sa[i] * su : 0.0f;
