@@ -1,5 +1,9 @@
 """The native caller of the C ABI (umdk_amd/_camcall.so) on the CPU: argument conversion, the library's errors, and the
 workspace it asks for.  Nothing launches: every call fails in its validation or in its allocation."""
+import shutil
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -59,3 +63,20 @@ def test_workspace_size_and_failed_allocation():
     with pytest.raises(MemoryError, match="no room"):
         raw("camhipDispatchLayout", 16, 64, 1, 8, 2, None, 16, None, 16, alloc=alloc)
     assert seen == [want]
+
+
+def test_calls_go_to_the_loaded_library(tmp_path):
+    # a library chosen through LIB_PATH (a diagnostic build) takes the calls too, and no other one is loaded
+    copy = tmp_path / "libother.so"
+    shutil.copy(_lib.LIB_PATH, copy)
+    code = f"""
+from umdk_amd import _lib
+_lib.LIB_PATH = {str(copy)!r}
+try:
+    _lib.call("camhipMoeRoute", None, None, 4, 8, 2, 16, 16, None, stream=0)
+except _lib.CamHipError as e:
+    assert "logits must not be NULL" in str(e)
+maps = open("/proc/self/maps").read()
+assert {str(copy)!r} in maps and "libcamhip.so" not in maps, "two libraries"
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=_lib._HERE + "/..")

@@ -1,5 +1,5 @@
 """Loader for libcamhip.so and a thin two-phase caller over its C ABI (the calls
-themselves in the extension module _camcall, built beside the library).
+themselves in the extension module _camcall, built beside the library and bound to the one loaded here).
 
 The library must already be built (``python -m umdk_amd.build`` or
 ``__graft_entry__.build()``); there is no fallback path: a missing library or
@@ -75,12 +75,12 @@ def lib():
 def _calls():
     global _caller
     if _caller is None:
-        lib()  # (its missing-library message first)
+        L = lib()  # (its missing-library message first)
         try:
             from . import _camcall
         except ImportError as e:
             raise ImportError(f"umdk_amd/_camcall.so is not built ({e}); run `python -m umdk_amd.build`") from e
-        _camcall.set_error(CamHipError)
+        _camcall.bind(L._handle, CamHipError)
         _caller = _camcall
     return _caller
 

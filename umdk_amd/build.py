@@ -4,7 +4,7 @@
 
 Every source is compiled by hipcc for gfx950 only; symbols are hidden except
 the extern "C" entry points declared in include/camhip.h.  _camcall.so is the
-Python caller of those entry points (host code, g++), linked against the library.
+Python caller of those entry points (host code, g++); it takes them from the library that _lib has loaded.
 """
 import os
 import subprocess
@@ -51,8 +51,7 @@ def _build_caller():
     tmp = CALLER + ".tmp"
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
            "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
-           os.path.join(HERE, "pyext", "camcall.cpp"), "-o", tmp, "-L" + LIBDIR, "-l:libcamhip.so",
-           "-Wl,-rpath,$ORIGIN/lib", "-Wl,--allow-shlib-undefined"]
+           os.path.join(HERE, "pyext", "camcall.cpp"), "-o", tmp, "-ldl"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("building _camcall.so failed:\n" + r.stdout + r.stderr)

@@ -8,9 +8,12 @@
 //   args: the GetWorkspaceSize arguments (pointers as int or None, sizes as any integer), without the two outputs;
 //   alloc: called with the workspace size when it is not 0, returns a tensor (its data_ptr is used and the tensor is
 //          returned); None: the caller's workspace is used;
-//   a failed call raises the exception set by set_error with the library's message.
+//   a failed call raises bind's exception with the library's message.
+// bind(handle, error): takes the entry points from an open library (a dlopen handle), the one its Python loader has
+// loaded; this module links to none, so a diagnostic build loaded in the library's place gets every call.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <dlfcn.h>
 
 #include <tuple>
 #include <type_traits>
@@ -21,6 +24,8 @@
 namespace {
 
 PyObject *g_error = nullptr;
+decltype(&camhipGetLastErrorMsg) g_last_error = nullptr;
+decltype(&camhipReleaseExecutor) g_release = nullptr;
 
 template <typename A> bool convert(PyObject *o, A &out)
 {
@@ -43,8 +48,8 @@ template <typename A> bool convert(PyObject *o, A &out)
 
 PyObject *failed(const char *name, const char *phase, int status)
 {
-    PyErr_Format(g_error ? g_error : PyExc_RuntimeError, "%s%s failed (%d): %s", name, phase, status,
-                 camhipGetLastErrorMsg());
+    PyErr_Format(g_error, "%s%s failed (%d): %s", name, phase, status,
+                 g_last_error());
     return nullptr;
 }
 
@@ -57,6 +62,10 @@ PyObject *invoke(const char *name, camhipStatus (*get)(P...), RunFn run, PyObjec
 {
     if (n != FIXED + (Py_ssize_t)sizeof...(I)) {
         PyErr_Format(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, (Py_ssize_t)sizeof...(I), n - FIXED);
+        return nullptr;
+    }
+    if (!g_error) {
+        PyErr_SetString(PyExc_RuntimeError, "_camcall is not bound to a library");
         return nullptr;
     }
     std::tuple<P...> a{};
@@ -82,7 +91,7 @@ PyObject *invoke(const char *name, camhipStatus (*get)(P...), RunFn run, PyObjec
         Py_XDECREF(p);
         if (!ok) {
             Py_XDECREF(buf);
-            camhipReleaseExecutor(ex);
+            g_release(ex);
             return nullptr;
         }
         have = (int64_t)need;
@@ -119,25 +128,45 @@ PyObject *entry(const char *name, camhipStatus (*get)(P...), RunFn run, PyObject
     X(camhipMoeExperts)
 
 #define DEFINE(f)                                                                                                    \
+    decltype(&f##GetWorkspaceSize) get_##f = nullptr;                                                                \
+    RunFn run_##f = nullptr;                                                                                         \
     PyObject *py_##f(PyObject *, PyObject *const *argv, Py_ssize_t n)                                                \
     {                                                                                                                \
         if (n < FIXED) {                                                                                             \
             PyErr_SetString(PyExc_TypeError, #f ": alloc, workspace, workspace_bytes and stream come first");        \
             return nullptr;                                                                                          \
         }                                                                                                            \
-        return entry(#f, f##GetWorkspaceSize, f, argv, n);                                                           \
+        return entry(#f, get_##f, run_##f, argv, n);                                                                 \
     }
 ENTRIES(DEFINE)
 
-PyObject *set_error(PyObject *, PyObject *type)
+template <typename F> bool resolve(void *lib, const char *name, F &out)
 {
+    out = (F)dlsym(lib, name);
+    if (!out)
+        PyErr_Format(PyExc_ImportError, "the library has no %s", name);
+    return out != nullptr;
+}
+
+PyObject *bind(PyObject *, PyObject *args)
+{
+    PyObject *handle, *type;
+    void *lib = nullptr;
+    if (!PyArg_ParseTuple(args, "OO", &handle, &type) || !convert(handle, lib))
+        return nullptr;
+#define RESOLVE(f)                                                                                                   \
+    if (!resolve(lib, #f "GetWorkspaceSize", get_##f) || !resolve(lib, #f, run_##f))                                 \
+        return nullptr;
+    ENTRIES(RESOLVE)
+    if (!resolve(lib, "camhipGetLastErrorMsg", g_last_error) || !resolve(lib, "camhipReleaseExecutor", g_release))
+        return nullptr;
     Py_INCREF(type);
     Py_XSETREF(g_error, type);
     Py_RETURN_NONE;
 }
 
 #define METHOD(f) {#f, (PyCFunction)(void (*)(void))py_##f, METH_FASTCALL, nullptr},
-PyMethodDef g_methods[] = {ENTRIES(METHOD){"set_error", set_error, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef g_methods[] = {ENTRIES(METHOD){"bind", bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_camcall", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
