@@ -1605,7 +1605,6 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
 {
     const int G = gridDim.x, bid = blockIdx.x;
     const int pos = (G & 7) ? bid : (bid & 7) * (G >> 3) + (bid >> 3);  // XCD-aware order
-    constexpr bool KEEP = ROLE != SYNC_NONE;
     constexpr bool HAS32 = DT != DT_INT8;
     // tiles of each class (uniform values read from LDS go to scalar registers at once: a VGPR holding one across
     // the classes gets spilled, and its reload after a tile's k-loop makes the next k-loop wait for it at every
@@ -1697,58 +1696,58 @@ __device__ __forceinline__ void big_schedule(const GmmArgs &p, const GroupTables
         light_queue(q);
         return;
     }
-    // Static plan: layer by layer, each layer one light tile for every block of the group (the free blocks, the others)
-    // that then ends first, counted in 20ths of a heavy tile's time.  A light tile's time against a heavy one's: 14/20 for
-    // a 128-row tile (measured 73 against 105 us in GMM1, 24 against 34 us in GMM2; int8 66 against 95 us), 11/20 and
-    // 5/20 for a 32-row tile with and without SwiGLU.  Within a group the tiles go round-robin, the sequence going on
-    // from class to class.
-    const int nbusy = ge - nfree, ng = is_free ? nfree : nbusy;
-    int busy_end = 20, free_end = 0, at = 0;
-    auto light = [&](int n, int cost, int &rs, int &rn) {
-        int nf = 0, nb = 0, layers = 0, last = 0;  // tiles of the free blocks, of the others; this group's layers
-        while (nf + nb < n) {
-            const bool f = nfree > 0 && (nbusy == 0 || free_end <= busy_end);
-            const int layer = min(n - nf - nb, f ? nfree : nbusy);
-            nf += f ? layer : 0;
-            nb += f ? 0 : layer;
-            free_end += f ? cost : 0;
-            busy_end += f ? 0 : cost;
-            layers += f == is_free;
-            last = f == is_free ? layer : last;
-        }
-        // (only a group's last layer can be partial)
-        const int r = rank >= ng ? G_NOWHERE : rank >= at ? rank - at : rank - at + ng;
-        rs = __builtin_amdgcn_readfirstlane((is_free ? 0 : nf) + r);
-        rn = __builtin_amdgcn_readfirstlane(r < last ? layers : r < ng ? max(layers - 1, 0) : 0);
-        at = __builtin_amdgcn_readfirstlane(at + last >= ng ? at + last - ng : at + last);
-        free_end = __builtin_amdgcn_readfirstlane(free_end);
-        busy_end = __builtin_amdgcn_readfirstlane(busy_end);
-    };
-    int rs, rn;
     if constexpr (ROLE == SYNC_NONE) {
+        // Static plan: layer by layer, each layer one light tile for every block of the group (the free blocks, the others)
+        // that then ends first, counted in 20ths of a heavy tile's time.  A light tile's time against a heavy one's: 14/20 for
+        // a 128-row tile (measured 73 against 105 us in GMM1, 24 against 34 us in GMM2; int8 66 against 95 us), 11/20 and
+        // 5/20 for a 32-row tile with and without SwiGLU.  Within a group the tiles go round-robin, the sequence going on
+        // from class to class.
+        const int nbusy = ge - nfree, ng = is_free ? nfree : nbusy;
+        int busy_end = 20, free_end = 0, at = 0;
+        auto light = [&](int n, int cost, int &rs, int &rn) {
+            int nf = 0, nb = 0, layers = 0, last = 0;  // tiles of the free blocks, of the others; this group's layers
+            while (nf + nb < n) {
+                const bool f = nfree > 0 && (nbusy == 0 || free_end <= busy_end);
+                const int layer = min(n - nf - nb, f ? nfree : nbusy);
+                nf += f ? layer : 0;
+                nb += f ? 0 : layer;
+                free_end += f ? cost : 0;
+                busy_end += f ? 0 : cost;
+                layers += f == is_free;
+                last = f == is_free ? layer : last;
+            }
+            // (only a group's last layer can be partial)
+            const int r = rank >= ng ? G_NOWHERE : rank >= at ? rank - at : rank - at + ng;
+            rs = __builtin_amdgcn_readfirstlane((is_free ? 0 : nf) + r);
+            rn = __builtin_amdgcn_readfirstlane(r < last ? layers : r < ng ? max(layers - 1, 0) : 0);
+            at = __builtin_amdgcn_readfirstlane(at + last >= ng ? at + last - ng : at + last);
+            free_end = __builtin_amdgcn_readfirstlane(free_end);
+            busy_end = __builtin_amdgcn_readfirstlane(busy_end);
+        };
+        int rs, rn;
         if (halve) {
             gmm_body<DT, EPI, CLS_128M, ROLE, false, W_CACHED, true>(p, gt, G_NOWHERE, place_among(blocks_for(2 * r)), 1, G, wv,
                                                                      TileQueue{}, n0 - r);
             return;
         }
-    }
-    if (n1 > 0) {
-        light(n1, 14, rs, rn);
-        gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
-        lds_sync();
-    }
-    if constexpr (DT == DT_INT8) {
-        if (n2 > 0) {
-            light(n2, 14, rs, rn);
-            gmm_body<DT, EPI, CLS_128S, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+        if (n1 > 0) {
+            light(n1, 14, rs, rn);
+            gmm_body<DT, EPI, CLS_128M, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+            lds_sync();
         }
-    }
-    if constexpr (HAS32) {
-        if (n3 > 0) {
-            light(n3, EPI == EPI_PLAIN ? 5 : 11, rs, rn);
-            if (!KEEP && wv >= Tile<32>::NWAVES)
-                return;  // the 32-row tile's four waves go on (a barrier only counts the waves still running)
-            gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+        if constexpr (DT == DT_INT8) {
+            if (n2 > 0) {
+                light(n2, 14, rs, rn);
+                gmm_body<DT, EPI, CLS_128S, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+            }
+        }
+        if constexpr (HAS32) {
+            if (n3 > 0) {
+                light(n3, EPI == EPI_PLAIN ? 5 : 11, rs, rn);
+                if (wv >= Tile<32>::NWAVES)
+                    return;  // the 32-row tile's four waves go on (a barrier only counts the waves still running)
+                gmm_body<DT, EPI, CLS_32, ROLE>(p, gt, G_NOWHERE, rs, rn, ng, wv);
+            }
         }
     }
 }
@@ -1872,10 +1871,10 @@ template <typename K> static hipError_t set_lds(K kernel, size_t lds, int dev, s
     return e;
 }
 
-// Tile choice.  A row capacity of at most 48 rows per expert (decode) can only hold short
-// segments: the 32-row kernel.  Otherwise the 8-wave kernel, which picks the 128- or 256-row
-// tile on the device from the actual counts (a prefill-sized capacity may still hold short
-// segments when most rows are routed elsewhere).  One launch, no host synchronisation.
+// Tile choice.  A row capacity of at most 48 rows per expert on average (decode): the 4-wave kernel, 32- and 64-row tiles.
+// Otherwise the 8-wave kernel, which picks among 256-, 128- and 32-row tiles on the device from the actual counts (a
+// prefill-sized capacity may still hold short segments when most rows are routed elsewhere).  One launch, no host
+// synchronisation.
 template <int DT, int EPI> static hipError_t launch_one(GmmArgs a, hipStream_t s)
 {
     const int dev = current_device();
