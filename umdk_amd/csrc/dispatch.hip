@@ -155,9 +155,13 @@ __global__ __launch_bounds__(DISP_WAVES * 64) void dispatch_int8_kernel(
 // once, where a wave per token walks its destinations in turn, two passes over the row for each (128 tokens of 7168
 // columns, about one routed row each, and a shared expert, smooth scales: 6.1 us against 20 + 8.6 us that way).
 constexpr int DF_THREADS = 256, DF_NIT = 2;  // H <= 7168 <= 2 * 256 * 16
-// Without smooth scales up to this many picks (401 tokens of 1280 columns, 4 local picks each: 5.4 against 6.4 us); the
-// block per destination reads x once per pick, the wave per token once.
-constexpr int DF_MAX_TK = 4096;
+// Without smooth scales the block per destination quantises a token's row once per local pick, the wave per token once in
+// all.  One pick a token: the blocks always (4000 tokens of 7168 columns: 19.4 against 27.3 us).  More: up to as many picks
+// as the GPU runs at once.  All picks local, 8 a token, us of the blocks against the waves: 7168 columns 7.0 and 10.9 at
+// 1024 picks, 10.4 and 10.4 at 2048, 14.1 and 10.8 at 3072; 2048 columns 8.3 and 9.2 at 3072, 9.5 and 8.1 at 4096; 1024
+// columns 7.2 and 7.3 at 3072, 8.4 and 7.5 at 4096.  With half of 4 picks local, 7168 columns: 8.2 and 8.5 at 2048, 12.3
+// and 9.8 at 4096.
+static bool int8_by_dest(long T, int K, int H) { return K == 1 || T * K <= (H <= 2048 ? 3072 : 2048); }
 static_assert(DF_NIT * DF_THREADS * 16 >= DISP_NIT * 1024, "a row fits the block");
 __global__ __launch_bounds__(DF_THREADS) void dispatch_int8_dest_kernel(
     const uint16_t *__restrict__ x, const int32_t *__restrict__ topk_idx, const int32_t *__restrict__ send_offset,
@@ -313,7 +317,7 @@ hipError_t launch_dispatch(const uint16_t *x, const int32_t *topk_idx, const int
                            topk_idx, send_offset, rs, T, H, K, E, rank, cap, ex, scales, expand_idx, inv_out);
         break;
     case QUANT_INT8_FUSED:
-        if (smooth || share_smooth || (long)T * K <= DF_MAX_TK)
+        if (smooth || share_smooth || int8_by_dest(T, K, H))
             hipLaunchKernelGGL(dispatch_int8_dest_kernel, dim3((unsigned)T * (K + (share != nullptr))),
                                dim3(DF_THREADS), 0, s, x, topk_idx, send_offset, rs, T, H, K, E, rank, cap, ex, scales,
                                expand_idx, inv_out, smooth, share_smooth);
