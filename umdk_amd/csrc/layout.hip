@@ -195,8 +195,7 @@ __global__ __launch_bounds__(RANK_THREADS) void layout_rank_kernel(const IdxT *_
 // a scan launch, then ranks its own as layout_rank_kernel does; the last block also has the totals.  Measured in a graph,
 // against the three launches: T = 64, K = 8, E = 256: 3.5 against 7.1 us; T = 1021, K = 6, E = 160: 4.4 against 7.6 us;
 // T = 4096, K = 8, E = 256: 7.4 against 8.3 us, and two launches fewer for the host.  The work grows with the square of
-// the entries, and picks of one expert meet at one LDS counter, one at a time: a token's picks are distinct, so at most
-// T of them (32768 tokens that all pick one expert: 29 against 7 us).  Hence both limits.
+// the entries, and picks of one expert meet at one LDS counter, one at a time: hence both limits.
 constexpr int DIRECT_THREADS = 1024;
 constexpr int DIRECT_WAVES = DIRECT_THREADS / 64;
 constexpr int DIRECT_MAX = 32768, DIRECT_MAX_T = 4096;
@@ -209,22 +208,38 @@ __global__ __launch_bounds__(DIRECT_THREADS) void layout_direct_kernel(const Idx
     __shared__ int32_t wave_hist[DIRECT_WAVES][MAX_E];
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = blockIdx.x;
     const int i = c * DIRECT_THREADS + tid;
-    const int64_t own = i < TK ? (int64_t)topk_idx[i] : -1;
+    // (past the end: the chunk before's pick, for the wave's choice below)
+    const int64_t near = topk_idx[i < TK ? i : c > 0 ? i - DIRECT_THREADS : 0], own = i < TK ? near : -1;
     for (int j = tid; j < E; j += DIRECT_THREADS)
         base[j] = 0;
     for (int j = lane; j < E; j += 64)
         wave_hist[w][j] = 0;
     __syncthreads();
-    constexpr int U = 8;
-    for (int c0 = 0; c0 < c; c0 += U) {
-        int64_t v[U];
+    // f of every pick of the earlier chunks that names an expert, eight loads in flight a thread
+    auto earlier = [&](auto f) {
+        constexpr int U = 8;
+        for (int c0 = 0; c0 < c; c0 += U) {
+            int64_t v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            v[u] = topk_idx[(long)min(c0 + u, c - 1) * DIRECT_THREADS + tid];
+            for (int u = 0; u < U; ++u)
+                v[u] = topk_idx[(long)min(c0 + u, c - 1) * DIRECT_THREADS + tid];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (c0 + u < c && v[u] >= 0 && v[u] < E)
-                atomicAdd(&base[(int)v[u]], 1);
+            for (int u = 0; u < U; ++u)
+                if (c0 + u < c && v[u] >= 0 && v[u] < E)
+                    f((int)v[u]);
+        }
+    };
+    // A wave whose own picks all name one expert adds the agreeing ones of a wave together (32768 picks of one expert,
+    // within tokens too: 8 us, 29 us one at a time); the choice inside the loop cost ordinary picks 0.4 us.
+    if (__ballot((int)near == __builtin_amdgcn_readfirstlane((int)near)) != ~0ull) {
+        earlier([&](int e) { atomicAdd(&base[e], 1); });
+    } else {
+        earlier([&](int e) {
+            const uint64_t same = __ballot(e == __builtin_amdgcn_readfirstlane(e));
+            const bool in = (same >> lane) & 1;
+            if (!in || (same & lanemask_lt()) == 0)
+                atomicAdd(&base[e], in ? __popcll(same) : 1);
+        });
     }
     const bool valid = own >= 0 && own < E;
     const int e = valid ? (int)own : -1;
