@@ -8,7 +8,7 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "umdk_amd", "csrc")
 SOURCE = """
 #include "gmm_plan.h"
-extern "C" int rows32(int n32, int n64, int G) { return cam::small_rows32(n32, n64, G); }
+extern "C" int rows32(int n32, int n64, int tall, int G) { return cam::small_rows32(n32, n64, tall, G); }
 extern "C" int blocks(int n, int G) { return cam::plan_blocks(n, G); }
 extern "C" void gmm2(int b, int G, int t1, int ge, int t2, int c1, int c2, int *out)
 {
@@ -29,23 +29,26 @@ def plan(tmp_path_factory):
 
 
 def tiles(counts, ntn):
-    """32-row tiles of a GEMM with ntn N-tiles, and its tiles with 64-row ones for the experts of more than 32 rows."""
-    return (sum(-(-c // 32) for c in counts) * ntn,
-            sum(-(-c // 64) if c > 32 else -(-c // 32) for c in counts) * ntn)
+    """32-row tiles of a GEMM with ntn N-tiles, its tiles with 64-row ones for the experts of more than 32 rows, and these."""
+    tall = sum(-(-c // 64) for c in counts if c > 32)
+    return sum(-(-c // 32) for c in counts) * ntn, (tall + sum(0 < c <= 32 for c in counts)) * ntn, tall * ntn
 
 
 def test_64_row_tiles_only_where_they_save_rounds(plan):
     ragged = [20, 36, 62, 40, 66, 33, 40, 34, 15, 14, 53, 45, 22, 33, 28, 14]
-    n32, n64 = tiles(ragged, 18)  # 486 and 306 tiles on 256 blocks: two rounds either way
-    assert -(-n32 // 256) == -(-n64 // 256) == 2 and plan.rows32(n32, n64, 256)
+    n32, n64, tall = tiles(ragged, 18)  # 486 and 306 tiles on 256 blocks: two rounds either way
+    assert -(-n32 // 256) == -(-n64 // 256) == 2 and plan.rows32(n32, n64, tall, 256)
     assert not plan.rows32(*tiles([45] * 16, 32), 256)   # 1024 -> 512 tiles
     assert not plan.rows32(*tiles([47] * 8, 56), 256)    # 896 -> 448
     assert plan.rows32(*tiles([45] * 8, 16), 256)        # one round
     assert plan.rows32(*tiles([20] * 64, 56), 256)       # no expert of more than 32 rows
-    for n32 in range(1, 3000, 7):  # never more rounds, weighted by a 64-row tile's time
+    assert not plan.rows32(*tiles([4] * 32 + [128], 16), 256)  # 576 -> 544, three rounds either way, 32 of them tall
+    assert not plan.rows32(*tiles([20] * 48 + [45] * 14 + [70] * 2, 36), 256)  # twelve rounds to ten
+    for n32 in range(1, 3000, 7):  # rounds, a tall one weighted by a 64-row tile's time, unless few are tall
         for n64 in range(max(1, n32 // 2), n32 + 1, 13):
-            if not plan.rows32(n32, n64, 256):
-                assert 1.25 * -(-n64 // 256) <= -(-n32 // 256)
+            for tall in range(0, n64 + 1, 61):
+                if not plan.rows32(n32, n64, tall, 256):
+                    assert 4 * tall <= n64 or -(-n64 // 256) + 0.25 * -(-tall // 256) <= -(-n32 // 256)
 
 
 @pytest.mark.parametrize("G", [256, 304, 250])

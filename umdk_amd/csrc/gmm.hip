@@ -286,7 +286,7 @@ __device__ ClassTiles build_group_tables(const int64_t *__restrict__ group_list,
     }
     bool rows32 = false;
     if constexpr (FOUR_WAVES)  // slot 2 counts the M-tiles with 32-row tiles throughout (small_ranges)
-        rows32 = small_rows32(tot[2] * ntn, (tot[CLS_128M] + tot[CLS_32]) * ntn, (int)gridDim.x);
+        rows32 = small_rows32(tot[2] * ntn, (tot[CLS_128M] + tot[CLS_32]) * ntn, tot[CLS_128M] * ntn, (int)gridDim.x);
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
         const int e = tid * PER + q;

@@ -11,16 +11,18 @@
 namespace cam {
 
 // 32-row tiles throughout (n32 of them), or 64-row tiles for the experts of more than 32 rows (n64 tiles of both
-// heights)?  Blocks run their tiles one after another, so what counts is rounds over the G blocks, and a 64-row tile
-// takes 1.25 to 1.35 times a 32-row one (the plain GEMM of 16 fp8 experts of 14 to 66 rows, K = 1024, N = 2304: 306 tiles,
-// two rounds, 20.2 us, against 486 tiles, also two rounds, 15.5 us).  64-row tiles from a fifth fewer rounds on (8 experts
-// of 47 rows, H = 7168, I = 2048, four rounds to three in GMM2: fp8 88 against 103 us, int8 91 against 94 us at a
-// quarter, bf16 152 against 156 us).
-CAM_PLAN_FN bool small_rows32(int n32, int n64, int G)
+// heights, tall of them 64-row ones)?  Blocks run their tiles one after another, so what counts is rounds over the G
+// blocks, and a round of 64-row tiles takes 1.25 to 1.35 times as long (the plain GEMM of 16 fp8 experts of 14 to 66 rows,
+// K = 1024, N = 2304: 306 tiles, 198 tall, two rounds, 20.2 us, against 486 tiles, also two rounds, 15.5 us).  So 64-row
+// tiles where the rounds they save make up for theirs (8 experts of 47 rows, H = 7168, I = 2048, four rounds to three in
+// GMM2: int8 91 against 94 us, bf16 152 against 156 us; 64 fp8 experts of 24 rows on average, H = 1792, I = 4608, twelve to
+// ten: 281 against 287 us), and where few are tall, which then only spare the memory (32 int8 experts of a few rows and a
+// shared one of 128, H = 7168, I = 2048, three rounds either way: the decode step 264 against 272 us).
+CAM_PLAN_FN bool small_rows32(int n32, int n64, int tall, int G)
 {
-    if (n32 <= G)
+    if (n32 <= G || tall == 0)
         return true;
-    return n64 == n32 || 5 * ((n64 + G - 1) / G) > 4 * ((n32 + G - 1) / G);
+    return 4 * tall > n64 && 4 * ((n64 + G - 1) / G) + (tall + G - 1) / G > 4 * ((n32 + G - 1) / G);
 }
 
 // Blocks that share n equal tiles in whole rounds: with R = ceil(n / G) rounds, only the first ceil(n / R) blocks
