@@ -202,9 +202,13 @@ camhipStatus camhipFusedDeepMoeGetWorkspaceSize(
     const bool int8 = dt == cam::DT_INT8;
     const int N = T * K;
     // A shared expert of the routed experts' width joins their GEMMs as group L, its rows (every token) after the
-    // routed ones (128 tokens, 32 of 256 int8 experts, H = 7168, I = 2048, smooth scales: the decode step 272 us
-    // against 347 us with its own dispatch, GEMMs and requantisation); one of another width, and a batch past the
-    // single-launch layouts, keeps its own launches.
+    // routed ones; one of another width, and a batch past the single-launch layouts, keeps its own dispatch, GEMMs and
+    // requantisation.  Joined against own launches, us of a decode step: 32 of 256 experts, top-8, H = 7168, I = 2048: 64
+    // tokens fp8 212 and 271, bf16 395 and 501, int8 226 and 277; 177 tokens 267 and 333, 491 and 568, 291 and 335; 1024
+    // tokens 329 and 402, 580 and 675, 367 and 399.  1024 tokens, 256 experts, top-8, H = 2048, I = 512: 278 and 304, 457
+    // and 485, 310 and 335.  4096 tokens, 160 experts, top-1, H = 4096, I = 1024: 480 and 581, 840 and 884, 566 and 613.
+    // In the 57 sizes measured (8 to 4096 tokens, 8 to 256 experts) it is never slower.  The GEMMs choose their kernel by
+    // all rows, the T of this expert too; by the routed rows alone was no better (fp8, 177 tokens: 276 us, 4096: 602 us).
     const bool merged = shared && Ish == I && N <= 8192 && L < 512 &&
                         (int64_t)(N + T) * std::max(H, I) * (dt == cam::DT_BF16 ? 2 : 1) < (int64_t)1 << 32;
     const FusedLayout f = plan_fused(T, H, K, L, I, shared ? Ish : 0, dt, shared && !merged, merged);
