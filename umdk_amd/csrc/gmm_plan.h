@@ -49,7 +49,7 @@ CAM_PLAN_FN int plan_place(int b, int g, int G) { return (G & 7) ? b : b < g ? (
 // of its last round, or without any, are free: they come first.  In a last round of several a free block has about one
 // GMM1 tile's time, worth R GMM2 tiles (cost1 and cost2: the bytes of weights of a tile of either), but never more than
 // spreads GMM2's tiles over the free blocks.  In an only round no GMM2 tile can start before the others end, so one tile
-// each, then the other blocks in turn (64 tokens of 16 experts, H = 2304, I = 1024, 192 GMM1 tiles: the step 66 us fp8 and
+// each, then the other blocks in turn (64 tokens of 16 experts, H = 2304, I = 1024, 192 GMM1 tiles: the step 67 us fp8 and
 // 91 us bf16, against 87 and 110 us with runs of 5 on the free blocks; one token through 2 of 8 bf16 experts, H = 1024:
 // 16 GMM2 tiles on 16 blocks).
 struct ChainGmm2 {
