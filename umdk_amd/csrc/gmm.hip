@@ -107,8 +107,8 @@ template <int BM_, int BN_ = GBN> struct Tile {
 #endif
 constexpr int small_bn(int bm, int epi) { return bm <= 64 && epi == 0 ? CAM_GMM_SMALL_PLAIN_BN : GBN; }
 
-// Tile classes: 256-row tiles, 128-row tiles of experts with several of them, 128-row tiles of experts with one,
-// 32-row tiles; and in the 4-wave kernels, in the place of CLS_128M, 64-row tiles.  The two 128-row classes differ in
+// Tile classes: 256-row tiles; 128-row tiles; in int8 128-row tiles of experts of up to 32 rows, in fp8 and bf16 32-row
+// tiles of these; and in the 4-wave kernels, in the place of CLS_128M, 64-row tiles.  The two 128-row classes differ in
 // how they fetch their weights (see W_CACHED and W_STREAM).
 enum TileClass { CLS_256 = 0, CLS_128M = 1, CLS_128S = 2, CLS_32 = 3, CLS_64 = 4 };
 constexpr int G_NCLASS = 4;
@@ -432,11 +432,12 @@ struct TileQueue {
 // each: the 8-wave kernels have no registers for that).  An expert that fits one M-tile has its weights read exactly
 // once; the M-tiles of an expert of several, which the tile order runs side by side on one XCD, re-read them from that
 // XCD's L2 (48 experts of 36 to 281 rows, fp8, K = 4096, N = 2816: 173 us cached, 205 us nontemporal).  A stream past
-// the caches pays where it spares the lines that others re-read: the 4-wave decode tiles, and int8's single M-tiles,
-// beside heavy experts (the layer of 22 touched experts, one of 2311 rows: 382 us nontemporal, 405 us cached) and
-// without (weights that differ from call to call: the layer of 8 experts of 1 to 24 rows, H = 2304, I = 1792, 55.3
-// against 59.9 us cached; 16 experts of 2 to 194 rows, H = 4864, I = 512, 86.9 against 90.8 us).  fp8 and bf16 keep
-// their single M-tiles of more than 32 rows cached (48 experts of 100 rows: 160 against 158 us; a class less).
+// the caches pays for light tiles: the 4-wave decode tiles, and in the 8-wave kernels the experts of up to 32 rows (32-row
+// tiles; in int8 128-row ones).  int8, weights that differ from call to call, the layer of 8 experts of 1 to 24 rows,
+// H = 2304, I = 1792: 55.0 us, 60.3 us cached; 16 experts of 2 to 194 rows, H = 4864, I = 512: 78.3 us against 86.0 with
+// every single M-tile (up to 128 rows) streamed and 91.0 with none; the skewed layer of 22 touched experts, one of 2311
+// rows: 342.6 against 354.7 us with every single M-tile; 32 experts of 122 rows on average, H = 4352, I = 6784: 688
+// against 718 and 705 us.
 enum WPolicy { W_CACHED = 0, W_STREAM = 1, W_BY_TILE = 2 };
 // 64-row tiles in fp8, which has no registers for two loops: as a stream, also where an expert has several (the decode
 // step of 400 tokens, 64 experts, H = 2048, I = 1408 140 against 148 us cached; 32 experts of 44 rows, H = 4096,
@@ -1586,13 +1587,13 @@ __host__ __device__ constexpr bool big_tall(int allow256, int K, int dt)
 {
     return allow256 && (int)((uint32_t)K * (dt == DT_BF16 ? 2 : 1) / GKB) >= CAM_GMM_MIN_NK256;
 }
-// int8: the single 128-row tiles are a class of their own (fp8 and bf16 move their smallest experts to 32-row tiles
-// instead: one GEMM loop fewer in their kernels leaves the 256-row loop more registers)
+// int8: the experts of up to 32 rows are a class of 128-row tiles of their own, for the way it fetches weights (fp8 and bf16
+// give them 32-row tiles)
 template <int DT> __device__ __forceinline__ ClassRanges big_ranges(bool tall)
 {
     constexpr int SMALL = DT == DT_INT8 ? 1 : G_SMALL_ROWS;  // rows below: the 32-row tile class
     const int top = tall ? G_HEAVY_ROWS : 0x7fffffff, small = tall ? SMALL : 1;
-    const int multi = tall && DT == DT_INT8 ? 129 : small;
+    const int multi = tall && DT == DT_INT8 ? G_SMALL_ROWS : small;
     return ClassRanges{{top, multi, small, 1}, {0x7fffffff, top, multi, small}};
 }
 
