@@ -38,7 +38,9 @@ def call(ops, d, E, mask, sw, int8, weights=None):
 # decode sizes with the layout in the dispatch, the same at its limit (2048 picks), past it (8-wave GEMMs, wave-per-token
 # int8 rows above 3072 picks), and past the single-launch layouts (8192 picks), where the expert keeps its own launches
 SIZES = [(3, 1024, 128, 8, 2), (40, 2048, 256, 16, 4), (256, 1024, 256, 8, 8), (300, 1024, 256, 16, 8),
-         (600, 1024, 128, 8, 8), (1100, 1024, 128, 8, 8)]
+         (600, 1024, 128, 8, 8), (1100, 1024, 128, 8, 8),
+         # int8 rows by the block per destination and, one token on, by the wave per token: 3072 picks, 2048 of wide rows
+         (384, 1024, 128, 16, 8), (385, 1024, 128, 16, 8), (256, 2304, 128, 8, 8), (257, 2304, 128, 8, 8)]
 
 
 @pytest.mark.parametrize("kind", ["bf16", "fp8", "int8", "int8_smooth"])
